@@ -1,0 +1,520 @@
+"""The work a user of this library has it do, as cases that can be timed.
+
+A case is a plain dict.  `prepare` builds what a host program holds before the call (grid,
+deck, initial state, a context on the device), `run` is one pass through the public entry
+points with what it hands back, `work` the bytes and operations a pass cannot do without and
+`exact` an independent evaluation where one is short enough to write down.
+
+Kinds of pass:
+
+  march    a resident solve is advanced by `steps` pseudo-time iterations and its state is
+           read back into the host's arrays, as between two outputs of a solve
+  dropin   the reference's loop body call by call (spectral radius, BC, space, LU-SGS update
+           with its norms, history shift), `steps` times, then state, gradients and D are read
+  cascade  Runge-Kutta DES steps with running time statistics, then state and statistics
+  rhs      the residual as a right-hand side: a state is uploaded, the spectral radius and the
+           inviscid residual are formed, and D, Rds and the time step are read back
+  serve    a batch of independent solves submitted to the server and run to their iteration
+           limit, every final state collected
+  wall     the wall distance of a set of cell centres to a set of wall panels
+"""
+from __future__ import annotations
+
+import copy
+import ctypes as C
+import dataclasses
+import functools
+import math
+
+import numpy as np
+import torch
+
+from trans_amd import capi, cases, mesh, serving, solver
+from trans_amd.params import make_params
+
+STATE = ("v", "pp", "t", "rmiu")   # what an output routine reads
+HISTORY = ("wt0", "wt1")           # dual-time history, needed to go on from the state
+
+
+# ---------------------------------------------------------------------------------------
+# the cases
+
+def listed():
+    return [
+        # one iteration on a small channel, state handed back: launch and call latency
+        dict(name="bump_step", kind="march", grid="bump", ni=33, nj=17, nk=5, fp32=0, steps=1),
+        # the channel bump at its usual size, Euler, Roe + MUSCL, FP64 operator
+        dict(name="bump_march", kind="march", grid="bump", ni=129, nj=65, nk=9, fp32=0, steps=100),
+        # the turbulent flat plate, 8 uneven blocks: RANS-SST, MDCD + AUSMPW+, FP64 operator
+        dict(name="plate_march", kind="march", grid="plate", nblk=8, ni=257, nj=129, nk=5, fp32=0, steps=100),
+        # a small odd-sized plate with the FP32 implicit operator
+        dict(name="plate_odd_fp32", kind="march", grid="plate", nblk=3, ni=98, nj=66, nk=4, fp32=1, steps=50),
+        # a 127k-cell compressor sector, one block re-oriented, FP64 operator
+        dict(name="sector_fp64", kind="march", grid="sector", scale=0.25, crossed=1, fp32=0, steps=100),
+        # the 0.49M-cell sector of the serving family, FP32 operator
+        dict(name="sector_march", kind="march", grid="sector", scale=0.39, crossed=0, fp32=1, steps=150),
+        # the 2M-cell sector of the serving family, FP32 operator: the largest
+        dict(name="sector_large", kind="march", grid="sector", scale=0.63, crossed=0, fp32=1, steps=150),
+        # a Fortran-style host that calls the routines one by one and watches the norms
+        dict(name="sector_dropin", kind="dropin", grid="sector", scale=0.39, crossed=0, fp32=0, steps=40),
+        # the DES cascade: RK3, one global time step, running mean and RMS statistics
+        dict(name="cascade_stats", kind="cascade", scale=0.25, steps=25),
+        # inviscid residual of a host-side state, MUSCL + Roe
+        dict(name="bump_rhs", kind="rhs", ni=161, nj=81, nk=17),
+        # four small sectors at different back pressures through the server
+        dict(name="serve_sectors", kind="serve", scale=0.125, solves=4, iters=100),
+        # wall distance of a sector's cells to all of its wall panels
+        dict(name="wall_distance", kind="wall", cells=485_000, panels=30_000),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(("bump", "plate", "plate", "sector", "sector", "dropin", "cascade", "rhs", "serve", "wall"))
+    if kind == "bump":
+        return dict(kind="march", grid="bump", ni=_log_int(rng, 17, 161), nj=_log_int(rng, 9, 97),
+                    nk=_log_int(rng, 4, 17), fp32=rng.randint(0, 1), steps=_log_int(rng, 1, 100))
+    if kind == "plate":
+        nblk = rng.randint(2, 8)
+        return dict(kind="march", grid="plate", nblk=nblk, ni=nblk * rng.randint(16, 40) + 1,
+                    nj=_log_int(rng, 25, 129), nk=rng.randint(4, 9), fp32=rng.randint(0, 1),
+                    steps=_log_int(rng, 5, 100))
+    if kind in ("sector", "dropin"):
+        c = dict(kind="march" if kind == "sector" else "dropin", grid="sector",
+                 scale=round(math.exp(rng.uniform(math.log(0.0625), math.log(0.45))), 4), crossed=rng.randint(0, 1),
+                 fp32=rng.randint(0, 1), steps=_log_int(rng, 5, 60))
+        return c
+    if kind == "cascade":
+        return dict(kind="cascade", scale=round(rng.uniform(0.125, 0.28), 4), steps=rng.randint(2, 20))
+    if kind == "rhs":
+        return dict(kind="rhs", ni=_log_int(rng, 17, 161), nj=_log_int(rng, 9, 97), nk=_log_int(rng, 4, 21))
+    if kind == "serve":
+        return dict(kind="serve", scale=round(rng.uniform(0.0625, 0.16), 4), solves=rng.randint(2, 5),
+                    iters=rng.randint(20, 100))
+    return dict(kind="wall", cells=_log_int(rng, 1000, 485_000), panels=_log_int(rng, 100, 30_000))
+
+
+# ---------------------------------------------------------------------------------------
+# grids and states
+
+@functools.lru_cache(maxsize=6)
+def _grid(grid, *size):
+    """Blocks with connectivity and geometry, and the deck: they do not depend on the state."""
+    if grid == "bump":
+        blocks, org, glob = cases.bump_channel(*size)
+    elif grid == "plate":
+        nblk, ni, nj, nk = size
+        mean = (ni - 1) / nblk + 1  # uneven blocks around the mean extent
+        blocks, org, glob = cases.flat_plate(nblk=nblk, ni_total=ni, nj=nj, nk=nk, lo=max(5, int(0.5 * mean)),
+                                             hi=int(2.0 * mean))
+    elif grid == "sector":
+        scale, crossed = size
+        blocks, org, glob = cases.compressor_sector(scale=scale, crossed=bool(crossed))
+        # the deck's CFL ramp only serves the start of the 8M-cell grid
+        org.CFL_Sub_start = org.CFL_Sub_end = 2.0
+        org.CFL_Sub_step = 1
+    else:
+        (scale,) = size
+        blocks, org, glob = cases.cascade(scale=scale)
+    solver.prepare_case(blocks, org, glob, device_geometry=True)
+    return blocks, org, glob
+
+
+def _case_grid(case):
+    if case["kind"] == "cascade":
+        return _grid("cascade", case["scale"])
+    if case["kind"] == "serve":
+        return _grid("sector", case["scale"], 0)
+    grid = case.get("grid", "bump")
+    if grid == "sector":
+        return _grid("sector", case["scale"], case["crossed"])
+    if grid == "plate":
+        return _grid("plate", case["nblk"], case["ni"], case["nj"], case["nk"])
+    return _grid("bump", case["ni"], case["nj"], case["nk"])
+
+
+def _state(grid_blocks, org, prm, rng, amp):
+    """Blocks sharing the grid's geometry with a state of their own: the uniform start with
+    every cell disturbed by up to +-amp, p, T and rho*E consistent."""
+    blocks = []
+    for g in grid_blocks:
+        b = copy.copy(g)
+        b.arrays = dict(g.arrays)
+        blocks.append(b)
+    mesh.initial_state(blocks, prm, q_dst=org.Q_Dst, if_ns_uniform=org.IF_NS_Uniform)
+    for b in blocks:
+        V, PP, T = b["v"], b["pp"], b["t"]
+        shp = PP.shape
+
+        def noise():
+            return amp * np.asfortranarray(rng.random(shp[::-1]).T * 2.0 - 1.0)
+        r = V[0] * (1.0 + noise())
+        vel = [V[m] / V[0] + noise() for m in (1, 2, 3)]
+        p = PP * (1.0 + noise())
+        V[0] = r
+        for m in range(3):
+            V[m + 1] = r * vel[m]
+        PP[...] = p
+        V[4] = p / 0.4 + 0.5 * r * sum(u * u for u in vel) - 0.5 * (prm.omega1 * b["rad"]) ** 2 * r
+        T[...] = prm.rxm2 * p / r
+        if org.IF_Euler == 0:
+            V[5] *= 1.0 + noise()
+            V[6] *= 1.0 + noise()
+        for nm in ("wt0", "wt1"):
+            b[nm][...] = V
+    return blocks
+
+
+class _HostArrays:
+    """The host program's own block arrays: per field one buffer for all blocks, and the views
+    of each block's part (reference layout, bounds -2:N+2) that the library fills."""
+
+    def __init__(self, blocks, fields):
+        self.flat, self.views = {}, [dict() for _ in blocks]
+        for nm, nc in fields.items():
+            n = [nc * int(np.prod(b.shape())) for b in blocks]
+            buf = np.zeros(sum(n))
+            o = 0
+            for q, b in enumerate(blocks):
+                shp = b.shape() if nc == 1 else (nc,) + b.shape()
+                self.views[q][nm] = capi.fview(buf[o:o + n[q]].reshape(shp, order="F"))
+                o += n[q]
+            self.flat[nm] = buf
+
+    def state_view(self, blk):
+        s = capi.TransStateView()
+        for nm in ("v", "pp", "t", "rmiu", "wt0", "wt1", "wt2"):
+            if nm in self.views[blk]:
+                setattr(s, nm, self.views[blk][nm])
+        return s
+
+
+NCOMP = {"v": 7, "pp": 1, "t": 1, "rmiu": 1, "wt0": 7, "wt1": 7, "wt2": 7}
+
+
+def _check(sv, rc):
+    if rc != 0:
+        raise RuntimeError(f"trans_hip error {rc}: {sv.lib.trans_hip_last_error(sv.ctx).decode()}")
+
+
+def _read_state(sv, views):
+    for blk, v in enumerate(views):
+        _check(sv, sv.lib.trans_hip_get_state(sv.ctx, blk, C.byref(v)))
+
+
+def _read_fields(sv, host, which):
+    for blk, views in enumerate(host.views):
+        for nm, field in which.items():
+            _check(sv, sv.lib.trans_hip_get_field(sv.ctx, blk, field, C.byref(views[nm])))
+
+
+def _norms(resid):
+    return np.array([[r[k] for k in ("drsa", "dua", "drsk", "duk", "drso", "duo")] for r in resid])
+
+
+# ---------------------------------------------------------------------------------------
+# prepare
+
+def prepare(case, seed):
+    rng = np.random.Generator(np.random.PCG64(seed))
+    kind = case["kind"]
+    if kind == "wall":
+        return _prepare_wall(case, rng)
+    grid_blocks, org, glob = _case_grid(case)
+    if kind == "serve":
+        return _prepare_serve(case, grid_blocks, org, glob, rng)
+    prm = make_params(org, glob, implicit_fp32=case.get("fp32", 0))
+    blocks = _state(grid_blocks, org, prm, rng, 0.005)
+    st = {"case": case}
+    if kind == "cascade":
+        prm.dt_lusgs_main = cases.global_time_step(blocks, prm, org.CFL_Sub_end)
+    sv = st["sv"] = solver.Solver(blocks, prm, ki=1)
+    names = STATE + (("wt2",) if kind == "cascade" else HISTORY)
+    fields = {nm: NCOMP[nm] for nm in names}
+    if kind == "cascade":
+        sv.stats_enable(1, 1)
+        fields["stats"] = capi.NSTAT
+    elif kind == "dropin":
+        fields.update(d=7, dqdxyz=18)
+    elif kind == "rhs":
+        fields = {"d": 7, "rds": 3, "dtm": 1}
+        st["in"] = [mesh.state_view(b) for b in blocks]
+    st["host"] = _HostArrays(blocks, fields)
+    if kind != "rhs":
+        st["views"] = [st["host"].state_view(q) for q in range(len(blocks))]
+    return st
+
+
+def _prepare_serve(case, grid_blocks, org, glob, rng):
+    n = case["solves"]
+    requests = []
+    for q in range(n):
+        g = dataclasses.replace(glob, Pouthub=float(rng.uniform(0.9, 1.3)) * glob.P0in)
+        prm = make_params(org, g, implicit_fp32=1)
+        requests.append((_state(grid_blocks, org, prm, rng, 0.005), prm))
+    hosts = [_HostArrays(blocks, NCOMP) for blocks, _ in requests]
+    return {"case": case, "server": serving.Server(hbm_budget=32 << 30, max_active=8, chunk=25),
+            "requests": requests, "hosts": hosts,
+            "views": [[h.state_view(b) for b in range(len(grid_blocks))] for h in hosts]}
+
+
+def _wall_points(case, rng):
+    """Cell centres in a unit box above two walls, and the walls' panel centres."""
+    nc, npan = case["cells"], case["panels"]
+    cells = rng.random((nc, 3)) * np.array([3.0, 1.0, 0.5])
+    pan = rng.random((npan, 3)) * np.array([3.0, 0.0, 0.5])
+    pan[:, 1] = np.where(rng.random(npan) < 0.5, 0.05 * np.sin(pan[:, 0]), 1.0)
+    return cells, pan
+
+
+def _prepare_wall(case, rng):
+    cells, pan = _wall_points(case, rng)
+    return {"case": case, "cells": cells, "panels": pan}
+
+
+# ---------------------------------------------------------------------------------------
+# run
+
+def run(state):
+    case = state["case"]
+    return {"march": _run_march, "dropin": _run_dropin, "cascade": _run_cascade, "rhs": _run_rhs,
+            "serve": _run_serve, "wall": _run_wall}[case["kind"]](case, state)
+
+
+def _run_march(case, state):
+    sv, host = state["sv"], state["host"]
+    resid = sv.iterate(case["steps"])
+    _read_state(sv, state["views"])
+    return dict(host.flat, norms=_norms(resid))
+
+
+def _run_dropin(case, state):
+    sv, host = state["sv"], state["host"]
+    norms = []
+    for _ in range(case["steps"]):
+        sv.spectral_radius()
+        sv.bc(-1)
+        sv.space()
+        norms.append(_norms(sv.lusgs_update()))
+        sv.update_u()
+    _read_state(sv, state["views"])
+    _read_fields(sv, host, {"d": capi.FIELD_D, "dqdxyz": capi.FIELD_DQDXYZ})
+    return dict(host.flat, norms=np.stack(norms))
+
+
+def _run_cascade(case, state):
+    sv, host = state["sv"], state["host"]
+    resid = sv.iterate(case["steps"])
+    _read_state(sv, state["views"])
+    for blk, views in enumerate(host.views):
+        _check(sv, sv.lib.trans_hip_get_stats(sv.ctx, blk, C.byref(views["stats"])))
+    return dict(host.flat, norms=_norms(resid))
+
+
+def _run_rhs(case, state):
+    sv, host = state["sv"], state["host"]
+    for blk, v in enumerate(state["in"]):
+        _check(sv, sv.lib.trans_hip_set_state(sv.ctx, blk, C.byref(v)))
+    sv.spectral_radius()
+    sv.space()
+    _read_fields(sv, host, {"d": capi.FIELD_D, "rds": capi.FIELD_RDS, "dtm": capi.FIELD_DTM})
+    return dict(host.flat)
+
+
+def _run_serve(case, state):
+    srv = state["server"]
+    ids = [srv.submit(blocks, prm, target_drop=1e-30, max_iter=case["iters"]) for blocks, prm in state["requests"]]
+    srv.run()
+    out = []
+    for rid, host, views in zip(ids, state["hosts"], state["views"]):
+        for blk, v in enumerate(views):
+            rc = srv.lib.trans_srv_result(srv.srv, rid, blk, C.byref(v))
+            if rc:
+                raise RuntimeError(f"trans_srv_result: {rc}")
+        out.append(dict(host.flat, drsa=srv.poll(rid)["drsa_last"]))
+        srv.release(rid)
+    return out
+
+
+def _run_wall(case, state):
+    return mesh.wall_distance_device(state["cells"], state["panels"])
+
+
+# ---------------------------------------------------------------------------------------
+# work
+
+def work(case):
+    """Compulsory bytes and operations of a pass.  One iteration reads the state (v, p, T, mu_t,
+    wt0, wt1) and the geometry once and writes the state once, with one round trip of the
+    increment between the sweeps: 432 bytes per cell (376 with the FP32 operator), 270 without
+    turbulence, 416 per Runge-Kutta stage; what is handed back is written once (ghost layers are
+    not counted).  Operations per cell and iteration (FP64 adds,
+    multiplies, divisions and roots of the three directions' face fluxes, the gradients, the
+    sources and the sweeps), counted from the reference's expressions: about 1400 inviscid, 3600
+    RANS, 3000 per Runge-Kutta stage."""
+    kind = case["kind"]
+    if kind == "wall":
+        n, m = case["cells"], case["panels"]
+        return {"bytes": 8.0 * (4 * n + 3 * m), "flops": 8.0 * n * m}
+    cells = _cells(case)
+    if kind == "rhs":
+        return {"bytes": 8.0 * (10 * cells + (13 + 24 + 11) * cells), "flops": 1000.0 * cells}
+    if kind == "serve":
+        b = 376.0 * case["iters"] * cells + 8.0 * (31 + 31 + 23) * cells
+        return {"bytes": case["solves"] * b, "flops": case["solves"] * 3600.0 * case["iters"] * cells}
+    if kind == "cascade":
+        return {"bytes": (3 * 416.0 + 8 * 2 * capi.NSTAT) * case["steps"] * cells + 8.0 * (17 + capi.NSTAT) * cells,
+                "flops": 3 * 3000.0 * case["steps"] * cells}
+    euler = case["grid"] == "bump"
+    per = 270.0 if euler else (376.0 if case["fp32"] else 432.0)
+    out = 24 + (25 if kind == "dropin" else 0)
+    return {"bytes": per * case["steps"] * cells + 8.0 * out * cells,
+            "flops": (1400.0 if euler else 3600.0) * case["steps"] * cells}
+
+
+def _cells(case):
+    """Interior cells of a case's grid."""
+    kind = case["kind"]
+    if kind == "cascade":
+        s = case["scale"]
+        seg = [max(2, int(round(n * s))) for n in (64, 96, 96, 96, 128, 160)]
+        nk = max(4, int(round(64 * s)))
+        ns, np_ = max(4, 2 * int(round(16 * s))), max(8, 2 * int(round(224 * s)))
+        cells = nk * (sum(seg) * np_ + (sum(seg) - seg[1] - seg[2]) * ns)
+    elif kind == "serve" or case.get("grid") == "sector":
+        s = case["scale"]
+        n = max(8, 2 * int(round(64 * s)))
+        cells = sum(max(3, int(round(m * s))) for m in (48, 128, 128, 128, 64)) * n * n
+    else:
+        cells = (case["ni"] - 1) * (case["nj"] - 1) * (case["nk"] - 1)
+    return cells
+
+
+# ---------------------------------------------------------------------------------------
+# exact
+
+def exact(case, seed):
+    rng = np.random.Generator(np.random.PCG64(seed))
+    if case["kind"] == "wall":
+        cells, pan = _wall_points(case, rng)
+        return _exact_wall(cells, pan)
+    if case["kind"] == "rhs":
+        grid_blocks, org, glob = _case_grid(case)
+        prm = make_params(org, glob)
+        blocks = _state(grid_blocks, org, prm, rng, 0.005)
+        out = [_exact_rhs(b, org, prm) for b in blocks]
+        return {nm: np.concatenate([o[nm].ravel(order="F") for o in out]) for nm in ("d", "rds", "dtm")}
+    return None  # whole solves: many iterations of the full scheme
+
+
+def _exact_wall(cells, pan):
+    dev = "cuda" if torch.cuda.is_available() else "cpu"
+    c = torch.from_numpy(cells).to(dev)
+    p = torch.from_numpy(pan).to(dev)
+    best = torch.full((c.shape[0],), math.inf, dtype=torch.float64, device=dev)
+    step = max(1, 40_000_000 // max(1, p.shape[0]))
+    for s in range(0, c.shape[0], step):
+        d = c[s:s + step]
+        d2 = sum((d[:, None, x] - p[None, :, x]) ** 2 for x in range(3))
+        best[s:s + step] = d2.amin(dim=1)
+    return best.clamp_min(1e-20).sqrt().cpu().numpy()
+
+
+def _exact_rhs(b, org, prm):
+    """Spectral radii, local time step and the inviscid residual (MUSCL with the smooth limiter,
+    Roe with the fixed 0.1 entropy floor) of one block from the state's own ghost cells."""
+    o = mesh.O
+    n = (b.ni - 1, b.nj - 1, b.nk - 1)
+    V, PP, T, Al, sd = b["v"], b["pp"], b["t"], b["alagm"], b["sd"]
+
+    def box(a, axis=None, shift=0, extra=0):
+        """Interior cells of a, shifted along one axis and with `extra` more cells there."""
+        s = [slice(o + 1, o + 1 + m) for m in n]
+        if axis is not None:
+            s[axis] = slice(o + 1 + shift, o + 1 + shift + n[axis] + extra)
+        return a[tuple(s)]
+
+    prim = [V[1] / V[0], V[2] / V[0], V[3] / V[0], PP, T]
+    den, vol = box(V[0]), box(b["vol"])
+    vel = [box(q) for q in prim[:3]]
+    cs = np.sqrt(1.4 * box(PP) / den)
+    x = prm.csth1 * box(T)
+    mul = (1.0 + prm.csthlnd) / (x + prm.csthlnd) * x ** 1.5
+    mut = box(b["rmiu"])
+    visc = np.maximum((mul + mut + 1e-20) * 4.0 / 3.0, (mul / 0.72 + mut / 0.9 + 1e-20) * 1.4) / den
+    rds = np.zeros((3,) + b.shape())
+    dtm = np.zeros(b.shape())
+    d = np.zeros((7,) + b.shape())
+    inner = tuple(slice(o + 1, o + 1 + m) for m in n)
+    total = 0.0
+    for ax in range(3):
+        S = [0.5 * (box(sd[ax + 3 * m]) + box(sd[ax + 3 * m], ax, 1)) for m in range(3)]
+        s2 = sum(q * q for q in S)
+        r = np.abs(sum(u * q for u, q in zip(vel, S))) + np.sqrt(s2) * cs + 2.0 * s2 / vol * visc / prm.ref
+        rds[ax][inner] = r
+        total = total + r
+    dtm[inner] = org.CFL_Sub_end * vol / total
+
+    def limited(a, c):
+        e = 1e-7 * 1e-7
+        up = a * (c * c + 2 * e) + c * (2 * a * a + e)
+        same = 0.5 * np.abs(np.copysign(1.0, a) + np.copysign(1.0, c))
+        return up / (2 * a * a - a * c + 2 * c * c + 3 * e) * same
+
+    for ax in range(3):
+        al = [box(Al[ax], ax, m, 1) for m in (-2, -1, 0, 1)]
+
+        def mean(lo, q0, q1):
+            return (al[lo + 1] * q0 + al[lo] * q1) / (al[lo] + al[lo + 1])
+        L, R = [], []
+        for q in prim:
+            c = [box(q, ax, m, 1) for m in (-2, -1, 0, 1)]
+            fm, f0, fp = (mean(m, c[m], c[m + 1]) for m in range(3))
+            L.append(c[1] + limited(f0 - c[1], c[1] - fm))
+            R.append(c[2] - limited(c[2] - f0, fp - c[2]))
+        area = box(b["grad"][ax], ax, 0, 1)
+        nrm = [box(sd[ax + 3 * m], ax, 0, 1) / area for m in range(3)]
+        flux = _roe(L, R, nrm, prm.ppf)
+        first = [slice(None)] * 3
+        last = [slice(None)] * 3
+        first[ax], last[ax] = slice(0, -1), slice(1, None)
+        for m in range(5):
+            f = flux[m] * area
+            d[m][inner] += f[tuple(last)] - f[tuple(first)]
+    return {"d": d, "rds": rds, "dtm": dtm}
+
+
+def _roe(L, R, nrm, ppf):
+    """Minus the Roe flux per unit area through faces with unit normals nrm."""
+    g1 = 1.4 - 1.0
+
+    def side(q):
+        rho = q[3] / (ppf * q[4])
+        return rho, 1.4 * q[3] / (rho * g1) + 0.5 * sum(u * u for u in q[:3])
+    (rl, hl), (rr, hr) = side(L), side(R)
+    w = np.sqrt(rr / rl)
+    rm = np.sqrt(rr * rl)
+    um = [(a + c * w) / (1.0 + w) for a, c in zip(L[:3], R[:3])]
+    hm = (hl + hr * w) / (1.0 + w)
+    v2 = sum(u * u for u in um)
+    a2 = g1 * np.abs(hm - 0.5 * v2)
+    a = np.sqrt(a2)
+    un = sum(s * u for s, u in zip(nrm, um))
+    e1, e2, e3 = (np.where(e < 0.1, (e * e + 0.01) / 0.2, e) for e in (np.abs(un), np.abs(un + a), np.abs(un - a)))
+    dv = [c - q for c, q in zip(R[:3], L[:3])]
+    dun = sum(s * q for s, q in zip(nrm, dv))
+    dr, dp = rr - rl, R[3] - L[3]
+    astar, mstar = 0.5 * (e2 + e3), 0.5 * (e2 - e3) / a
+    du = mstar * dun + (astar - e1) * dp / rm / a2
+    dpr = mstar * dp + (astar - e1) * rm * dun
+    ul, ur = (rho * sum(s * u for s, u in zip(nrm, q[:3])) for rho, q in ((rl, L), (rr, R)))
+    out = [-0.5 * (ul + ur - (e1 * dr + du * rm))]
+    for m in range(3):
+        diss = e1 * (rm * dv[m] + dr * um[m]) + du * rm * um[m] + dpr * nrm[m]
+        out.append(-0.5 * (ul * L[m] + ur * R[m] + nrm[m] * (L[3] + R[3]) - diss))
+    de = dp / g1 + 0.5 * v2 * dr + rm * sum(u * q for u, q in zip(um, dv))
+    out.append(-0.5 * (ul * hl + ur * hr - (e1 * de + du * rm * hm + dpr * un)))
+    return out
