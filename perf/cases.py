@@ -53,8 +53,8 @@ def listed():
         dict(name="sector_fp64", kind="march", grid="sector", scale=0.25, crossed=1, fp32=0, steps=100),
         # the 0.49M-cell sector of the serving family, FP32 operator
         dict(name="sector_march", kind="march", grid="sector", scale=0.39, crossed=0, fp32=1, steps=150),
-        # the 2M-cell sector of the serving family, FP32 operator: the largest
-        dict(name="sector_large", kind="march", grid="sector", scale=0.63, crossed=0, fp32=1, steps=150),
+        # the full 8.1M-cell sector, FP32 operator: the largest
+        dict(name="sector_full", kind="march", grid="sector", scale=1.0, crossed=0, fp32=1, steps=50),
         # a Fortran-style host that calls the routines one by one and watches the norms
         dict(name="sector_dropin", kind="dropin", grid="sector", scale=0.39, crossed=0, fp32=0, steps=40),
         # the DES cascade: RK3, one global time step, running mean and RMS statistics
@@ -84,7 +84,7 @@ def draw(rng):
                     steps=_log_int(rng, 5, 100))
     if kind in ("sector", "dropin"):
         c = dict(kind="march" if kind == "sector" else "dropin", grid="sector",
-                 scale=round(math.exp(rng.uniform(math.log(0.0625), math.log(0.45))), 4), crossed=rng.randint(0, 1),
+                 scale=round(math.exp(rng.uniform(math.log(0.0625), math.log(0.8))), 4), crossed=rng.randint(0, 1),
                  fp32=rng.randint(0, 1), steps=_log_int(rng, 5, 60))
         return c
     if kind == "cascade":
