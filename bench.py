@@ -66,10 +66,15 @@ def alg_bytes(name, neq, fp32, dual_shift=True):
         # SD(9), Rds(3)
         "k_lusgs_line<fwd>": ("cell", r * (2 * neq + 2 + (3 if turb else 0) + 4 + 1 + 9 + 3)),
         "k_lusgs_line<bwd>": ("cell", r * (2 * neq + 2 + (3 if turb else 0) + 4 + 1 + 9 + 3)),
-        # tile wavefront: the same inputs and increments as the line march, every input read
-        # once (the mean-flow and k-omega tiles share 1/rho, u, v, w, SD means and Rds)
-        "k_lusgs_tile<fwd>": ("cell", r * (2 * neq + (5 if turb else 2) + 4 + 1 + 9 + 3)),
-        "k_lusgs_tile<bwd>": ("cell", r * (2 * neq + (5 if turb else 2) + 4 + 1 + 9 + 3)),
+        # tile wavefront: increments in and out, stept/F1, cvs/F1 (stept, cvs, 1/F1t for k-omega),
+        # gamma p/rho, u, v, w, face means (9), Rds(3), every input read once (the mean-flow and
+        # k-omega waves share the last 15)
+        "k_lusgs_wave<fwd>": ("cell", r * (2 * neq + (5 if turb else 2) + 4 + 9 + 3)),
+        "k_lusgs_wave<bwd>": ("cell", r * (2 * neq + (5 if turb else 2) + 4 + 9 + 3)),
+        # the inputs of k_lusgs_rhs_w and k_sst_rhs_w (what both read, once); the packets' values out
+        "k_wave_rhs": ("cell", d * (5 + 5 + 5 + 5 + 3 + 1 + 1 + (2 + 2 + 4 + 15 + 1 + 1 + 1 if turb else 0))
+                       + r * (5 + 2 + 1 + 3 + 3 + (5 if turb else 0))),
+        "k_wave_unskew": ("cell", (r + d) * neq),
         # D(5), V(5), Wt0(5), Wt1(5), Rds(3), Dtm, Vol in; 17 sweep inputs out in the operator's precision
         "k_lusgs_rhs_w": ("cell", d * (5 + 5 + 5 + 5 + 3 + 1 + 1) + r * 17),
         "k_sst_rhs_w": ("cell", d * (2 + 3 + 2 + 2 + 15 + 1 + 1 + 1 + 1 + 3 + 1) + r * 3),

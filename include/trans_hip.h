@@ -34,7 +34,7 @@ extern "C" {
 #define TRANS_ENOMEM (-3)
 #define TRANS_EUNSUPPORTED (-4)
 #define TRANS_ESCRATCH (-5) /* input larger than a static staging array (trans_geom_wall_distance_static) */
-#define TRANS_ETIMEOUT (-6) /* a bounded wait of the tile-wavefront sweep expired (results invalid) */
+#define TRANS_ETIMEOUT (-6) /* a bounded wait of the wave sweeps expired (results invalid) */
 #define TRANS_ENONFINITE 1 /* a residual norm came out NaN (Time/TIME_Update_V.F90:124-151) */
 
 /*
@@ -200,9 +200,9 @@ typedef struct trans_ctx trans_ctx;
  * kernels' 32-bit per-block indexing (more than 2^28 padded cells). */
 int trans_hip_create(const trans_params* params, int nblk, const trans_block_desc* blocks,
                      trans_ctx** out);
-/* (The LU-SGS sweeps run as a line march when every block's cross-section fits one workgroup,
- * else as a hyperplane wavefront; TRANS_HIP_LINE_SWEEP=0 in the environment at create time
- * selects the hyperplane wavefront for all blocks.  Both give the same results.) */
+/* (The LU-SGS sweeps run as a wavefront of tiles of lines along j; TRANS_HIP_LINE_SWEEP=0 in the
+ * environment at create time selects one workgroup per block walking its hyperplanes.  Both give
+ * the same results.) */
 int trans_hip_destroy(trans_ctx* ctx);
 const char* trans_hip_last_error(const trans_ctx* ctx);
 
@@ -310,9 +310,9 @@ int trans_tecplot_write_ascii(const char* path, const char* title, const char* z
 
 /* ---- Launch autotuner (no counterpart in the reference) ------------------------------------
  * Times `iters` iterations of every launch configuration of the context from the same saved
- * state and keeps the fastest: the LU-SGS sweep (sweep = 0, 1, 2: line march along i, j or k,
- * where the cross sections fit one workgroup; 3: tile wavefront over many CUs with the tile
- * shapes tile_a x tile_b and progress chunks below; -2: one launch per hyperplane over all
+ * state and keeps the fastest: the LU-SGS sweep (sweep = 0, 2: line march along i or k, where the
+ * cross sections fit one workgroup; 1, where the (i, k) sections do, and 3, for all blocks: the
+ * wavefront of tiles of lines along j; -2: one launch per hyperplane over all
  * blocks; -1: one workgroup per block walking its hyperplanes), helper streams for the
  * face kernels (streams = 4) or one stream (1), HIP-graph replay (graph = 1) or eager launches.
  * Every configuration computes the same iteration (the sweep variants contract multiply-adds
@@ -321,13 +321,13 @@ int trans_tecplot_write_ascii(const char* path, const char* title, const char* z
  * buffer is reallocated for the chosen axis, so the context's device bytes may then differ
  * from trans_hip_footprint's.  get_tuning reports the configuration in use. */
 typedef struct trans_tune_entry {
-    int sweep;     /* 0, 1, 2 line march along i, j, k; 3 tile wavefront; -2 one launch per hyperplane;
+    int sweep;     /* 0, 2 line march along i, k; 1, 3 tile wavefront along j; -2 one launch per hyperplane;
                       -1 one workgroup per block; -3 plain drop-in schedule (set_tuning only) */
     int streams;
     int graph;
     double ms_per_iter;
-    int tile_a, tile_b; /* sweep 3: lines of a tile along i and along k (tile_a * tile_b <= 256) */
-    int chunk;          /* sweep 3: steps between a tile's progress stores */
+    int tile_a, tile_b; /* sweep 3: checked (tile_a * tile_b <= 256) and reported; a tile is 16 x 4 lines */
+    int chunk;          /* sweep 3: checked (positive) and reported; a tile hands every row on */
 } trans_tune_entry;
 int trans_hip_autotune(trans_ctx* ctx, int iters, trans_tune_entry* out, int max_out, int* n_out);
 int trans_hip_get_tuning(const trans_ctx* ctx, trans_tune_entry* out);
@@ -339,7 +339,7 @@ int trans_hip_get_tuning(const trans_ctx* ctx, trans_tune_entry* out);
  * hyperplane per block), on one stream, without graph replay; the same arithmetic as the
  * batched schedule.  Decks without preconditioning only (TRANS_EUNSUPPORTED otherwise).  A
  * baseline for the batched schedule; autotune leaves it for the batched candidates.
- * A tile-wavefront sweep whose progress wait exceeds its spin limit (a schedule that cannot
+ * A tile-wavefront sweep whose wait for another tile exceeds its spin limit (a schedule that cannot
  * advance) ends and makes the next synchronising call return TRANS_ETIMEOUT. */
 int trans_hip_set_tuning(trans_ctx* ctx, const trans_tune_entry* t);
 

@@ -19,6 +19,8 @@ struct BlkInfo {
     int patch0;      // first entry of this block in the device patch table
     long mwoff;      // offset of the block's wall marks in Fields::mw
     long woff;       // offset of the block in the hyperplane-major sweep buffer Fields::W
+    long poff;       // first element of the block's tile packets in Fields::P
+    long eoff;       // first element of the block's edge rows in a sweep's edge buffer
 };
 
 // One workgroup's share of an index space: block `blk`, linear indices base..base+255.
@@ -71,6 +73,7 @@ struct Fields {
     long wtot;        // component stride: the slots of all blocks, then the sinks
     long wsink;       // first sink slot (idle lanes of the line sweep store there)
     int march;        // march axis of the line sweep (0 i, 1 j, 2 k)
+    void* P;          // tile packets of the wave sweeps (k_wave.h; double or float), else null
 };
 
 // components of Fields::W / Fields::Wf (the line-march mean-flow sweep reads the step sizes

@@ -22,7 +22,7 @@ static bool rec_read(FILE* fp, void* data, size_t bytes)
 static BlkInfo blk_info(const trans_ctx* c, int blk)
 {
     const HostBlock& h = c->hb[blk];
-    return BlkInfo{h.ni, h.nj, h.nk, h.nx, h.ny, h.nz, h.off, 0, 0, 0, 0};
+    return BlkInfo{h.ni, h.nj, h.nk, h.nx, h.ny, h.nz, h.off, 0, 0, 0, 0, 0, 0};
 }
 
 // field (ncomp components, stride tot) of block blk <-> host vector in record order

@@ -23,8 +23,8 @@
 #include "k_space.h"
 #include "k_rk.h"
 #include "k_time.h"
-#include "k_tile.h"
 #include "k_visc.h"
+#include "k_wave.h"
 
 namespace {
 
@@ -108,15 +108,16 @@ struct trans_ctx {
     int max_planes = 0;
     void* wbuf = nullptr;  // the sweep buffer W / Wf (reallocated when the march axis changes)
     size_t wbytes = 0;
-    // tile wavefront of the sweeps (sweep mode 3, march axis j): tile tables for NEQ = 7, 5
-    // and 2 (mean flow and k-omega, mean flow alone, k-omega alone), the tiles' edge buffers,
-    // the item and progress counters of both sweeps, and the error flag of the bounded waits
-    bool tile_mode = false;
-    int tile_a = 16, tile_b = 16, tile_chunk = 8;
-    int tile_grid_k[3] = {0, 0, 0};  // persistent grid of the tile kernel for tables 0, 1, 2
-    SweepTile* d_tiles[3] = {nullptr, nullptr, nullptr};
-    int ntiles[3] = {0, 0, 0};
-    void* tile_edge = nullptr;
+    // wave sweeps (k_wave.h; sweep modes 1 and 3): the tile table, both sweeps' edge rows, their
+    // item counters, and the error flag of the bounded waits
+    bool wave = false;
+    bool wave_alt = false;  // round as the line march, which these blocks fit
+    int sweep_mode = -1;  // the mode asked for (cur_sweep)
+    int tile_a = 16, tile_b = 16, tile_chunk = 8;  // of the last set_tuning
+    WaveTile* d_tiles = nullptr;
+    int ntiles = 0;
+    void* wave_edge = nullptr;  // forward, then backward
+    long edge_n = 0;            // elements of one sweep's edge rows
     int* d_tctr = nullptr;
     size_t tile_bytes = 0;
     int* d_err = nullptr;
@@ -406,156 +407,89 @@ static bool march_fits(const trans_ctx* c, int m, int* mx_out)
     return mx <= 1024 && 4 * std::min(neq, (size_t)5) * (mx + 2) * esz <= 128 * 1024;
 }
 
-// Per-block descriptors (with each block's first slot in the sweep buffer) to the device.
+// Packet rows of a block's wave tiles.
+static long wave_block_rows(const HostBlock& h) { return (long)wave_nta(h.ni) * wave_ntb(h.nk) * wave_rows(h.nj); }
+
+// Per-block descriptors (with each block's first slot in the sweep buffers) to the device.
 static int upload_blk_table(trans_ctx* c)
 {
     const int nblk = (int)c->hb.size();
     std::vector<BlkInfo> bi(nblk);
-    long wt = 0;
+    long wt = 0, rows = 0;
     for (int b = 0; b < nblk; b++) {
         const HostBlock& h = c->hb[b];
         const int n[3] = {h.ni - 1, h.nj - 1, h.nk - 1};
         bi[b] = BlkInfo{h.ni, h.nj, h.nk, h.nx, h.ny, h.nz, h.off, c->patch0[b + 1] - c->patch0[b], c->patch0[b],
-                        c->mwoff[b], c->wbytes ? wt : 0};
+                        c->mwoff[b], c->wbytes ? wt : 0, rows * WaveRow<double>::ELEMS, rows * WaveEdge<double>::ELEMS};
         wt += (long)(n[0] + n[1] + n[2] - 2) * n[(c->march + 1) % 3] * n[(c->march + 2) % 3];
+        rows += wave_block_rows(h);
     }
     if (!c->d_blk) return 0;  // set before the table exists: create uploads it
     return h2d(c, c->d_blk, bi.data(), nblk * sizeof(BlkInfo));
 }
 
-// The sweep in use: 0, 1, 2 line march along that axis, 3 tile wavefront, -2 one launch per
-// hyperplane, -1 one workgroup per block.
-static int cur_sweep(const trans_ctx* c)
-{
-    if (c->plain) return -3;
-    if (c->tile_mode) return 3;
-    return c->line_threads ? c->march : (c->plane_launch ? -2 : -1);
-}
+// The sweep in use: 0, 2 line march along that axis, 1 and 3 the wave sweeps along j, -2 one launch
+// per hyperplane, -1 one workgroup per block.
+static int cur_sweep(const trans_ctx* c) { return c->plain ? -3 : c->sweep_mode; }
 
 static void free_tiles(trans_ctx* c)
 {
     if (!c->dry) {
-        for (SweepTile*& t : c->d_tiles)
-            if (t) (void)hipFree(t);
-        if (c->tile_edge) (void)hipFree(c->tile_edge);
+        if (c->d_tiles) (void)hipFree(c->d_tiles);
+        if (c->wave_edge) (void)hipFree(c->wave_edge);
         if (c->d_tctr) (void)hipFree(c->d_tctr);
     }
-    for (SweepTile*& t : c->d_tiles) t = nullptr;
-    for (int& n : c->ntiles) n = 0;
-    c->tile_edge = nullptr;
+    c->d_tiles = nullptr;
+    c->ntiles = 0;
+    c->wave_edge = nullptr;
+    c->edge_n = 0;
     c->d_tctr = nullptr;
     c->bytes -= c->tile_bytes;
     c->tile_bytes = 0;
 }
 
-// Tile tables of the wavefront sweep for the current tile shape (tile_a x tile_b lines):
-// table 0 holds the mean-flow and k-omega tiles, 1 the mean-flow ones, 2 the k-omega ones,
-// each in the order of the tiles' diagonals (upstream tiles first).  Edge buffers are laid
-// out once for table 0; the other tables use the same offsets.
+// Tile table of the wave sweeps in the order of the tiles' diagonals (upstream tiles first), the
+// edge rows of both sweeps and their item counters.
 static int build_tiles(trans_ctx* c)
 {
-    const int TA = c->tile_a, TB = c->tile_b;
-    if (TA < 1 || TB < 1 || TA * TB > TILE_MAXT) return fail(c, TRANS_EINVAL, "tile shape must have 1..256 lines");
     const size_t esz = c->p.implicit_fp32 ? sizeof(float) : sizeof(double);
-    struct Item {
-        int diag, blk, neq, ta, tb;
-    };
-    std::vector<Item> all;
+    std::vector<WaveTile> tab;
+    long rows = 0;
     for (int b = 0; b < (int)c->hb.size(); b++) {
         const HostBlock& h = c->hb[b];
-        const int nta = (h.ni - 1 + TA - 1) / TA, ntb = (h.nk - 1 + TB - 1) / TB;
-        for (int tb = 0; tb < ntb; tb++)
-            for (int ta = 0; ta < nta; ta++)
-                for (int neq : {5, 2}) all.push_back(Item{ta + tb, b, neq, ta, tb});
+        for (int tb = 0; tb < wave_ntb(h.nk); tb++)
+            for (int ta = 0; ta < wave_nta(h.ni); ta++) tab.push_back(WaveTile{b, ta, tb});
+        rows += wave_block_rows(h);
     }
-    std::stable_sort(all.begin(), all.end(), [](const Item& x, const Item& y) {
-        if (x.diag != y.diag) return x.diag < y.diag;
-        if (x.blk != y.blk) return x.blk < y.blk;
-        return x.neq > y.neq;
-    });
-    // edge offsets (elements), per (block, kind, ta, tb), from the full table
-    std::map<std::tuple<int, int, int, int>, std::pair<long, long>> eoff;
-    long etot = 0;
-    for (const Item& it : all) {
-        const HostBlock& h = c->hb[it.blk];
-        const int na = std::min(TA, h.ni - 1 - it.ta * TA), nb = std::min(TB, h.nk - 1 - it.tb * TB);
-        const long ea = etot;
-        etot += (long)it.neq * (h.nj - 1) * nb;
-        const long eb = etot;
-        etot += (long)it.neq * (h.nj - 1) * na;
-        eoff[std::make_tuple(it.blk, it.neq, it.ta, it.tb)] = std::make_pair(ea, eb);
-    }
-    int ntmax = 0;
-    std::vector<SweepTile> tab[3];
-    for (int w = 0; w < 3; w++) {
-        std::map<std::tuple<int, int, int, int>, int> index;
-        for (const Item& it : all) {
-            if ((w == 1 && it.neq != 5) || (w == 2 && it.neq != 2)) continue;
-            const HostBlock& h = c->hb[it.blk];
-            SweepTile t{};
-            t.blk = it.blk;
-            t.neq = it.neq;
-            t.a0 = it.ta * TA;
-            t.b0 = it.tb * TB;
-            t.na = std::min(TA, h.ni - 1 - t.a0);
-            t.nb = std::min(TB, h.nk - 1 - t.b0);
-            const auto& e = eoff[std::make_tuple(it.blk, it.neq, it.ta, it.tb)];
-            t.ea = e.first;
-            t.eb = e.second;
-            index[std::make_tuple(it.blk, it.neq, it.ta, it.tb)] = (int)tab[w].size();
-            tab[w].push_back(t);
-        }
-        for (SweepTile& t : tab[w]) {
-            const int ta = t.a0 / TA, tb = t.b0 / TB;
-            auto find = [&](int a, int b) {
-                auto q = index.find(std::make_tuple(t.blk, t.neq, a, b));
-                return q == index.end() ? -1 : q->second;
-            };
-            t.lo_a = find(ta - 1, tb);
-            t.hi_a = find(ta + 1, tb);
-            t.lo_b = find(ta, tb - 1);
-            t.hi_b = find(ta, tb + 1);
-        }
-        c->ntiles[w] = (int)tab[w].size();
-        ntmax = std::max(ntmax, c->ntiles[w]);
-    }
-    const size_t ctr_n = 2 + 2 * (size_t)ntmax;
-    const size_t bytes = 3 * (size_t)ntmax * sizeof(SweepTile) + (size_t)std::max(etot, 1L) * esz + ctr_n * sizeof(int);
-    c->tile_bytes = bytes;
-    c->bytes += bytes;
+    std::stable_sort(tab.begin(), tab.end(),
+                     [](const WaveTile& x, const WaveTile& y) { return x.ta + x.tb < y.ta + y.tb; });
+    c->ntiles = (int)tab.size();
+    c->edge_n = rows * WaveEdge<double>::ELEMS;
+    const size_t ebytes = 2 * (size_t)c->edge_n * esz;
+    c->tile_bytes = tab.size() * sizeof(WaveTile) + ebytes + 2 * sizeof(int);
+    c->bytes += c->tile_bytes;
     if (c->dry) return 0;
-    for (int w = 0; w < 3; w++) {
-        HIPCHK(c, hipMalloc(&c->d_tiles[w], std::max<size_t>(1, tab[w].size()) * sizeof(SweepTile)));
-        if (!tab[w].empty()) {
-            int rc = h2d(c, c->d_tiles[w], tab[w].data(), tab[w].size() * sizeof(SweepTile));
-            if (rc) return rc;
-        }
-    }
-    HIPCHK(c, hipMalloc(&c->tile_edge, (size_t)std::max(etot, 1L) * esz));
-    HIPCHK(c, hipMemsetAsync(c->tile_edge, 0, (size_t)std::max(etot, 1L) * esz, c->stream));
-    HIPCHK(c, hipMalloc(&c->d_tctr, ctr_n * sizeof(int)));
-    HIPCHK(c, hipMemsetAsync(c->d_tctr, 0, ctr_n * sizeof(int), c->stream));
-    // persistent grid: as many tile workgroups as the device holds at once
-    int dev = 0, cus = 0, occ = 0;
-    HIPCHK(c, hipGetDevice(&dev));
-    HIPCHK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    for (int w = 0; w < 3; w++) {
-        const void* kern;
-        if (c->p.implicit_fp32)
-            kern = w == 0 ? (const void*)k_lusgs_tile<float, true, 0>
-                          : (w == 1 ? (const void*)k_lusgs_tile<float, true, 5> : (const void*)k_lusgs_tile<float, true, 2>);
-        else
-            kern = w == 0 ? (const void*)k_lusgs_tile<double, true, 0>
-                          : (w == 1 ? (const void*)k_lusgs_tile<double, true, 5> : (const void*)k_lusgs_tile<double, true, 2>);
-        HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, TILE_MAXT, 0));
-        c->tile_grid_k[w] = std::max(1, std::min(TILE_GRID_MAX, std::max(1, occ) * std::max(1, cus)));
-    }
-    return 0;
+    HIPCHK(c, hipMalloc(&c->d_tiles, tab.size() * sizeof(WaveTile)));
+    HIPCHK(c, hipMalloc(&c->wave_edge, ebytes));
+    HIPCHK(c, hipMalloc(&c->d_tctr, 2 * sizeof(int)));
+    return h2d(c, c->d_tiles, tab.data(), tab.size() * sizeof(WaveTile));
 }
 
-// Selects the LU-SGS sweep: m = 0, 1, 2 the line march along that axis (hyperplane-major
-// buffer W or Wf, reallocated here), m = 3 the tile wavefront (march axis j), m = -2 one
-// launch per hyperplane, m = -1 the hyperplane kernel on the natural layout.
+// Face means of every block's interior cells (in the natural layout, and in the sweep buffer).
+static void launch_face_means(trans_ctx* c, int seg0, int nseg)
+{
+    const Seg* seg = c->seg_cell.d + seg0;
+    if (c->wave && c->p.implicit_fp32)
+        hipLaunchKernelGGL(k_wave_geom<float>, dim3(nseg), dim3(WG), 0, c->stream, c->f, c->d_blk, seg);
+    else if (c->wave)
+        hipLaunchKernelGGL(k_wave_geom<double>, dim3(nseg), dim3(WG), 0, c->stream, c->f, c->d_blk, seg);
+    else
+        hipLaunchKernelGGL(k_face_means, dim3(nseg), dim3(WG), 0, c->stream, c->f, c->d_blk, seg);
+}
+
+// Selects the LU-SGS sweep: m = 1 or 3 the wave sweeps along j (tile packets), m = 0 or 2 the line
+// march along that axis (hyperplane-major buffer W or Wf), m = -2 one launch per hyperplane (the
+// same buffer, march axis j), m = -1 the hyperplane kernel on the natural layout.
 static int set_sweep(trans_ctx* c, int m, bool upload)
 {
     int mx = 0;
@@ -563,13 +497,8 @@ static int set_sweep(trans_ctx* c, int m, bool upload)
     if (c->p.if_precondition && m != -1)
         return fail(c, TRANS_EUNSUPPORTED, "with IF_PRECONDITION = 1 only the hyperplane sweep (-1) runs");
     if (m < -2 || m > 3) return fail(c, TRANS_EINVAL, "sweep must be -2, -1, 0, 1, 2 or 3");
-    const bool planes = m == -2;  // per-plane launches on the hyperplane-major buffer, march axis j
-    const bool tiles = m == 3;    // tile wavefront on the hyperplane-major buffer, march axis j
-    if (planes || tiles) m = 1;
-    if (!planes && !tiles && m >= 0 && !march_fits(c, m, &mx))
+    if (m >= 0 && m <= 2 && !march_fits(c, m, &mx))
         return fail(c, TRANS_EINVAL, "the line sweep does not fit this axis");
-    c->plane_launch = planes;
-    c->tile_mode = tiles;
     free_tiles(c);
     if (c->wbuf) {
         if (!c->dry) (void)hipFree(c->wbuf);
@@ -580,54 +509,64 @@ static int set_sweep(trans_ctx* c, int m, bool upload)
     Fields& f = c->f;
     f.W = nullptr;
     f.Wf = nullptr;
+    f.P = nullptr;
     c->line_threads = 0;
-    if (m >= 0) {
-        c->march = m;
-        c->max_lines = mx;
-        c->line_threads = (planes || tiles) ? 0 : (mx + 63) / 64 * 64;
+    c->wave = false;
+    c->plane_launch = false;
+    c->sweep_mode = -1;
+    const size_t esz = c->p.implicit_fp32 ? sizeof(float) : sizeof(double);
+    if (m != -1) {
+        c->march = m == 0 || m == 2 ? m : 1;
         // hyperplane-major sweep buffer: nplanes x nlines slots per block, then per
         // component a sink of 1024 slots for each of the 2 workgroups of every block
-        long wt = 0;
+        long wt = 0, rows = 0;
+        bool rows_ok = true;  // a wave addresses its tile's rows with 31-bit byte offsets
         for (const HostBlock& h : c->hb) {
             const int n[3] = {h.ni - 1, h.nj - 1, h.nk - 1};
-            wt += (long)(n[0] + n[1] + n[2] - 2) * n[(m + 1) % 3] * n[(m + 2) % 3];
+            wt += (long)(n[0] + n[1] + n[2] - 2) * n[(c->march + 1) % 3] * n[(c->march + 2) % 3];
+            rows += wave_block_rows(h);
+            rows_ok = rows_ok && (long)wave_rows(h.nj) * WaveRow<double>::BYTES < (1L << 31);
         }
         f.wsink = wt;
-        // (the tile wavefront's persistent workgroups have TILE_MAXT sink slots each)
-        wt += tiles ? std::max((long)c->hb.size() * 2 * 1024, (long)TILE_GRID_MAX * TILE_MAXT)
-                    : (long)c->hb.size() * 2 * 1024;
+        wt += (long)c->hb.size() * 2 * 1024;
         // the sweep addresses a component with 32-bit byte offsets
-        if (wt * (long)sizeof(double) >= (1L << 32)) {
-            c->line_threads = 0;
-            c->plane_launch = false;
-            c->tile_mode = false;
+        if (wt * (long)sizeof(double) >= (1L << 32))
             return fail(c, TRANS_EUNSUPPORTED, "too many cells for the line-march sweep buffer");
+        c->wave = (m == 1 || m == 3) && rows_ok;
+        c->wave_alt = march_fits(c, 0, nullptr) || march_fits(c, 1, nullptr) || march_fits(c, 2, nullptr);
+        c->plane_launch = m == -2 || ((m == 1 || m == 3) && !rows_ok);
+        if (m == 0 || m == 2) {
+            c->max_lines = mx;
+            c->line_threads = (mx + 63) / 64 * 64;
         }
         f.wtot = wt;
-        f.march = m;
-        const size_t bytes = (size_t)W_NCOMP * wt * (c->p.implicit_fp32 ? sizeof(float) : sizeof(double));
+        f.march = c->march;
+        const size_t bytes = c->wave ? (size_t)rows * WaveRow<double>::ELEMS * esz : (size_t)W_NCOMP * wt * esz;
         if (!c->dry) {
             hipError_t e = hipMalloc(&c->wbuf, bytes);
             if (e != hipSuccess) return fail(c, TRANS_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-            HIPCHK(c, hipMemsetAsync(c->wbuf, 0, bytes, c->stream));
+            if (!c->wave) HIPCHK(c, hipMemsetAsync(c->wbuf, 0, bytes, c->stream));
         }
         c->wbytes = bytes;
         c->bytes += bytes;
-        if (c->p.implicit_fp32)
+        if (c->wave)
+            f.P = c->wbuf;
+        else if (c->p.implicit_fp32)
             f.Wf = (float*)c->wbuf;
         else
             f.W = (double*)c->wbuf;
     }
-    if (tiles) {
+    if (c->wave) {
         int rc = build_tiles(c);
         if (rc) return rc;
     }
+    c->sweep_mode = m;
     drop_graph(c);
     if (!upload) return 0;
     int rc = upload_blk_table(c);
-    if (rc || m < 0 || c->dry) return rc;
-    // the geometry part of the new buffer (face means W_SDM, written once per geometry upload)
-    hipLaunchKernelGGL(k_face_means, dim3(c->seg_cell.n), dim3(WG), 0, c->stream, c->f, c->d_blk, c->seg_cell.d);
+    if (rc || m == -1 || c->dry) return rc;
+    // the geometry part of the new buffer (face means, written once per geometry upload)
+    launch_face_means(c, 0, c->seg_cell.n);
     HIPCHK(c, hipGetLastError());
     return 0;
 }
@@ -770,16 +709,12 @@ static int create_ctx(const trans_params* params, int nblk, const trans_block_de
     if (!bs.empty() && (rc = h2d(c, c->d_bcseg, bs.data(), bs.size() * sizeof(BcSeg)))) return rc;
 
     {
-        // march along j (lanes on i: coalesced) unless the (i,k) sections do not fit a workgroup;
-        // TRANS_HIP_LINE_SWEEP=0 in the environment, or preconditioning, selects the hyperplane
+        // the wave sweeps along j; TRANS_HIP_LINE_SWEEP=0 in the environment, or preconditioning, selects the hyperplane
         // sweep instead
         const char* env = std::getenv("TRANS_HIP_LINE_SWEEP");
         const bool lines_ok = !(env && env[0] == '0') && !c->p.if_precondition;
-        const int order[3] = {1, 2, 0};
         int m = -1;
-        for (int q = 0; q < 3 && lines_ok && m < 0; q++)
-            if (march_fits(c, order[q], nullptr)) m = order[q];
-        if (lines_ok && m < 0) m = 3;  // blocks too large for a line-march workgroup: the tile wavefront
+        if (lines_ok) m = march_fits(c, 1, nullptr) ? 1 : 3;  // both run the wave sweeps
         if ((rc = set_sweep(c, m, false))) return rc;
     }
     if ((rc = dalloc(c, &c->d_blk, nblk))) return rc;
@@ -958,7 +893,7 @@ int trans_hip_set_geometry(trans_ctx* c, int blk, const trans_geom_view* g)
             mw.insert(mw.end(), (size_t)fsz[q], 0);
     }
     if ((rc = h2d(c, f.mw + c->mwoff[blk], mw.data(), mw.size() * sizeof(int)))) return rc;
-    hipLaunchKernelGGL(k_face_means, dim3(c->seg_cell.n), dim3(WG), 0, c->stream, c->f, c->d_blk, c->seg_cell.d);
+    launch_face_means(c, c->seg_cell.wrange[blk], c->seg_cell.wrange[blk + 1] - c->seg_cell.wrange[blk]);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return 0;
@@ -1180,8 +1115,6 @@ static void launch_lines(trans_ctx* c, R* dq)
 {
     if (c->march == 0)
         launch_lines<R, NEQ, MAXT, 0>(c, dq);
-    else if (c->march == 1)
-        launch_lines<R, NEQ, MAXT, 1>(c, dq);
     else
         launch_lines<R, NEQ, MAXT, 2>(c, dq);
 }
@@ -1198,21 +1131,6 @@ static void launch_sweeps(trans_ctx* c, R* dq)
             launch_lines<R, NEQ, 512>(c, dq);
         else
             launch_lines<R, NEQ, 1024>(c, dq);
-    } else if (c->tile_mode) {
-        const int w = NEQ == 7 ? 0 : (NEQ == 5 ? 1 : 2);
-        const int nt = c->ntiles[w];
-        const int ntmax = std::max(c->ntiles[0], std::max(c->ntiles[1], c->ntiles[2]));
-        const int nctr = 2 + 2 * ntmax;
-        const int grid = std::max(1, std::min(c->tile_grid_k[w], nt));
-        R* edge = (R*)c->tile_edge;
-        KLAUNCH(c, "k_tile_reset", k_tile_reset, dim3((nctr + 255) / 256), dim3(256), c->d_tctr, nctr);
-        constexpr int KIND = NEQ == 7 ? 0 : NEQ;
-        KLAUNCH(c, "k_lusgs_tile<fwd>", (k_lusgs_tile<R, true, KIND>), dim3(grid), dim3(TILE_MAXT), c->f, dq,
-                c->d_blk, c->d_tiles[w], nt, c->d_tctr, c->d_tctr + 2, edge, c->d_err, c->tile_chunk,
-                TILE_SPIN_LIMIT);
-        KLAUNCH(c, "k_lusgs_tile<bwd>", (k_lusgs_tile<R, false, KIND>), dim3(grid), dim3(TILE_MAXT), c->f, dq,
-                c->d_blk, c->d_tiles[w], nt, c->d_tctr + 1, c->d_tctr + 2 + ntmax, edge, c->d_err, c->tile_chunk,
-                TILE_SPIN_LIMIT);
     } else if (c->plane_launch) {
         const bool kw = NEQ == 2;
         for (int s0 = 0; s0 < c->max_planes; s0++)
@@ -1230,6 +1148,52 @@ static void launch_sweeps(trans_ctx* c, R* dq)
     }
 }
 
+// Both wave sweeps with PD packet rows in flight and registers for WPE waves per SIMD.
+template <typename R, int NEQ, bool ALT, int PD, int WPE>
+static void launch_wave_sweeps(trans_ctx* c)
+{
+    const dim3 grid(c->ntiles), blk(NEQ == 7 ? 128 : 64);
+    const bool kw = NEQ == 2;
+    R* edge = (R*)c->wave_edge;
+    KLAUNCH(c, kw ? "k_turb_wave<fwd>" : "k_lusgs_wave<fwd>", (k_lusgs_wave<R, true, NEQ, PD, WPE, ALT>), grid, blk,
+            c->f, c->d_blk, c->d_tiles, c->ntiles, c->d_tctr, edge, c->d_err, WV_SPIN_LIMIT);
+    KLAUNCH(c, kw ? "k_turb_wave<bwd>" : "k_lusgs_wave<bwd>", (k_lusgs_wave<R, false, NEQ, PD, WPE, ALT>), grid, blk,
+            c->f, c->d_blk, c->d_tiles, c->ntiles, c->d_tctr + 1, edge + c->edge_n, c->d_err, WV_SPIN_LIMIT);
+}
+
+// From four tiles per CU on (1024) the FP32 sweeps keep four rows of a wave in flight at two waves
+// per SIMD: 1169 us for both sweeps of the 8.1M-cell sector (1760 tiles, k-omega) instead of
+// 1307 us with two rows at four waves.  Below, a row's latency counts more than its loads: 179 us
+// against 201 us at 0.49M cells (392 tiles), 132 us against 134 us on a 25 k-cell plate (25 tiles).
+// The FP64 k-omega sweeps alone have the registers for a third row (334 us against 414 us for the
+// three stages of a 0.30M-cell cascade); with the mean flow two rows are as good (103 us against
+// 113 us at 0.13M cells).
+template <typename R, int NEQ, bool ALT>
+static void launch_wave_rule(trans_ctx* c)
+{
+    if constexpr (sizeof(R) == 8)
+        launch_wave_sweeps<R, NEQ, ALT, NEQ == 2 ? 3 : 2, 2>(c);
+    else if (c->ntiles >= 1024)
+        launch_wave_sweeps<R, NEQ, ALT, 4, 2>(c);
+    else
+        launch_wave_sweeps<R, NEQ, ALT, 2, 4>(c);
+}
+
+// Packet inputs, both wave sweeps and the increments back to D for NEQ = 7, 5 or 2 equations.
+template <typename R, int NEQ>
+static void launch_wave(trans_ctx* c)
+{
+    const bool kw = NEQ == 2;
+    KLAUNCH(c, "k_wave_rhs", (k_wave_rhs<R, NEQ != 2, NEQ != 5>), dim3(c->seg_wtile.n), dim3(WG), c->p, c->f, c->d_blk,
+            c->seg_wtile.d, c->d_tctr, (uint4*)c->wave_edge, (long)(2 * (size_t)c->edge_n * sizeof(R) / 16));
+    if (c->wave_alt)
+        launch_wave_rule<R, NEQ, true>(c);
+    else
+        launch_wave_rule<R, NEQ, false>(c);
+    KLAUNCH(c, "k_wave_unskew", k_wave_unskew<R>, dim3(c->seg_wtile.n), dim3(WG), kw ? 5 : 0, NEQ, c->f, c->d_blk,
+            c->seg_wtile.d);
+}
+
 extern "C" {
 
 // LU-SGS (Time/TIME_LUSGS.F90, Time/TURBTWO_TIME_LUSGS_SST.F90) and Update_V (main.F90:135-150)
@@ -1239,7 +1203,17 @@ static int lusgs_update_async(trans_ctx* c, int shift = 0)
     const int if_turb = if_turb_now(c);
     // the sweep buffer along j moves through LDS tiles (whole cache lines per diagonal)
     const bool wtiled = (c->f.W || c->f.Wf) && c->f.march == 1;
-    if (wtiled && c->f.Wf)
+    const int neq = if_turb ? 7 : 5;
+    if (c->wave) {
+        if (c->p.implicit_fp32 && if_turb)
+            launch_wave<float, 7>(c);
+        else if (c->p.implicit_fp32)
+            launch_wave<float, 5>(c);
+        else if (if_turb)
+            launch_wave<double, 7>(c);
+        else
+            launch_wave<double, 5>(c);
+    } else if (wtiled && c->f.Wf)
         KLAUNCH(c, "k_lusgs_rhs_w", k_lusgs_rhs_w<float>, dim3(c->seg_wtile.n), dim3(WG), c->p, c->f, c->d_blk,
                 c->seg_wtile.d);
     else if (wtiled)
@@ -1247,16 +1221,17 @@ static int lusgs_update_async(trans_ctx* c, int shift = 0)
                 c->seg_wtile.d);
     else
         KLAUNCH(c, "k_lusgs_rhs", k_lusgs_rhs, dim3(c->seg_cell.n), dim3(WG), c->p, c->f, c->d_blk, c->seg_cell.d);
-    if (if_turb) {
+    if (if_turb && !c->wave) {
         if (wtiled)
             KLAUNCH(c, "k_sst_rhs_w", k_sst_rhs_w, dim3(c->seg_wtile.n), dim3(WG), c->p, c->f, c->d_blk,
                     c->seg_wtile.d);
         else
             KLAUNCH(c, "k_sst_rhs", k_sst_rhs, dim3(c->seg_cell.n), dim3(WG), c->p, c->f, c->d_blk, c->seg_cell.d);
     }
-    const int neq = if_turb ? 7 : 5;
-    if (c->f.W || c->f.Wf) {
-        // line-march sweeps on the hyperplane-major buffer, increments back to D after
+    if (c->wave) {
+        // done: the increments are in D
+    } else if (c->f.W || c->f.Wf) {
+        // sweeps on the hyperplane-major buffer, increments back to D after
         if (c->p.implicit_fp32) {
             if (if_turb)
                 launch_sweeps<float, 7>(c, c->f.Wf);
@@ -1309,17 +1284,24 @@ static int rk_update_async(trans_ctx* c, int stage)
     const int if_turb = if_turb_now(c);
     // the sweep buffer along j moves through LDS tiles (whole cache lines per diagonal)
     const bool wtiled = (c->f.W || c->f.Wf) && c->f.march == 1;
-    KLAUNCH(c, "k_rk_stage", k_rk_stage, dim3(c->seg_cell.n), dim3(WG), c->p, stage, if_turb ? 0 : 1, wtiled ? 0 : 1,
+    KLAUNCH(c, "k_rk_stage", k_rk_stage, dim3(c->seg_cell.n), dim3(WG), c->p, stage, if_turb ? 0 : 1, wtiled || c->wave ? 0 : 1,
             c->f, c->d_blk, c->seg_cell.d, c->d_part);
     if (if_turb) {
-        if (wtiled) {
+        if (c->wave) {
+            if (c->p.implicit_fp32)
+                launch_wave<float, 2>(c);
+            else
+                launch_wave<double, 2>(c);
+        } else if (wtiled) {
             KLAUNCH(c, "k_rk_w", k_rk_w, dim3(c->seg_wtile.n), dim3(WG), c->p, c->f, c->d_blk, c->seg_wtile.d);
             KLAUNCH(c, "k_sst_rhs_w", k_sst_rhs_w, dim3(c->seg_wtile.n), dim3(WG), c->p, c->f, c->d_blk,
                     c->seg_wtile.d);
         } else {
             KLAUNCH(c, "k_sst_rhs", k_sst_rhs, dim3(c->seg_cell.n), dim3(WG), c->p, c->f, c->d_blk, c->seg_cell.d);
         }
-        if (c->f.W || c->f.Wf) {
+        if (c->wave) {
+            // done: the increments are in D
+        } else if (c->f.W || c->f.Wf) {
             if (c->p.implicit_fp32) {
                 launch_sweeps<float, 2>(c, c->f.Wf);
                 if (wtiled)
@@ -1363,7 +1345,7 @@ static int check_sweep_flag(trans_ctx* c)
     if (!e) return 0;
     HIPCHK(c, hipMemsetAsync(c->d_err, 0, sizeof(int), c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    return fail(c, TRANS_ETIMEOUT, "a bounded wait of the tile-wavefront LU-SGS sweep expired; results are invalid");
+    return fail(c, TRANS_ETIMEOUT, "a bounded wait of the wave LU-SGS sweep expired; results are invalid");
 }
 
 static int fetch_resid(trans_ctx* c, trans_resid* per_block)
@@ -1700,7 +1682,7 @@ int trans_hip_plane_integrals(trans_ctx* c, int blk, int dir, int index, trans_p
     const HostBlock& h = c->hb[blk];
     const int n = dir == 1 ? h.ni : (dir == 2 ? h.nj : h.nk);
     if (index < 1 || index > n) return fail(c, TRANS_EINVAL, "face index out of range");
-    BlkInfo b{h.ni, h.nj, h.nk, h.nx, h.ny, h.nz, h.off, 0, 0, 0, 0};
+    BlkInfo b{h.ni, h.nj, h.nk, h.nx, h.ny, h.nz, h.off, 0, 0, 0, 0, 0, 0};
     KLAUNCH(c, "k_plane_integrals", k_plane_integrals, dim3(1), dim3(256), c->f, b, dir, index, c->p.omega1,
             c->d_mon);
     double r[6];
