@@ -95,12 +95,11 @@ static int copy_between(const trans_fview& src, const trans_fview& dst)
     const long dn0 = dst.hi[0] - dst.lo[0] + 1, dn1 = dst.hi[1] - dst.lo[1] + 1;
     const int nc = src.ncomp;
     for (int k = lo[2]; k <= hi[2]; k++)
-        for (int j = lo[1]; j <= hi[1]; j++)
-            for (int i = lo[0]; i <= hi[0]; i++) {
-                const long si = (long)nc * ((i - src.lo[0]) + sn0 * ((j - src.lo[1]) + sn1 * (long)(k - src.lo[2])));
-                const long di = (long)nc * ((i - dst.lo[0]) + dn0 * ((j - dst.lo[1]) + dn1 * (long)(k - dst.lo[2])));
-                for (int c = 0; c < nc; c++) dst.p[di + c] = src.p[si + c];
-            }
+        for (int j = lo[1]; j <= hi[1]; j++) {  // a row of cells is contiguous in both
+            const long si = (long)nc * ((lo[0] - src.lo[0]) + sn0 * ((j - src.lo[1]) + sn1 * (long)(k - src.lo[2])));
+            const long di = (long)nc * ((lo[0] - dst.lo[0]) + dn0 * ((j - dst.lo[1]) + dn1 * (long)(k - dst.lo[2])));
+            std::memcpy(dst.p + di, src.p + si, (size_t)nc * (size_t)(hi[0] - lo[0] + 1) * sizeof(double));
+        }
     return 0;
 }
 
