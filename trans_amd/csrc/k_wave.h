@@ -534,9 +534,15 @@ __device__ __forceinline__ void wave_sweep(const Fields& f, const BlkInfo& b, in
             // refresh the rows already loaded
             const int tau = FORWARD ? s : nrow - 1 - s;
             for (int spins = 0;; spins++) {
+                // the next row's as well: a wave that follows its upstream tile that closely would
+                // otherwise poll on every row
                 bool pend = false;
 #pragma unroll
-                for (int L = 0; L < NEQ; L++) pend |= wv_pending<R>(x.ea[L]) | wv_pending<R>(x.eb[L]);
+                for (int r = 0; r < 2; r++) {
+                    const WaveIn<R, NEQ>& y = ring[(Q + r) % PD];
+#pragma unroll
+                    for (int L = 0; L < NEQ; L++) pend |= wv_pending<R>(y.ea[L]) | wv_pending<R>(y.eb[L]);
+                }
                 if (!__any(pend)) break;
                 if (spins > spin_limit ||
                     ((spins & 63) == 63 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
