@@ -45,14 +45,11 @@ def alg_bytes(name, neq, fp32, dual_shift=True):
         "k_prim_cells": ("cell", d * ((6 if turb else 4) + (5 if turb else 3))),
         # Q(3[,5]), T, Alagm(3), SD(9), Vol in; DQ(12[,18]), shock out
         "k_gradients": ("cell", d * ((5 if turb else 3) + 1 + 3 + 9 + 1 + (18 if turb else 12) + 1)),
-        # per face of direction d: cell Q(5), V(1), T, Rmiu, Dst, Alagm, Vol, DQ(18) once; SD(3); GV(6) out
-        "k_visc_face<1>": ("face1", d * (6 + 1 + 1 + 1 + 1 + 1 + 18 + 3 + 6)),
-        "k_visc_face<2>": ("face2", d * (6 + 1 + 1 + 1 + 1 + 1 + 18 + 3 + 6)),
-        "k_visc_face<3>": ("face3", d * (6 + 1 + 1 + 1 + 1 + 1 + 18 + 3 + 6)),
-        # per face: cell Q(3[,5]), V(1), PP, T, rad, Alagm, shock once; SD(3), Grad; G(5[,7]) out
-        "k_conv_face<1>": ("face1", d * ((6 if turb else 4) + 5 + 4 + (7 if turb else 5))),
-        "k_conv_face<2>": ("face2", d * ((6 if turb else 4) + 5 + 4 + (7 if turb else 5))),
-        "k_conv_face<3>": ("face3", d * ((6 if turb else 4) + 5 + 4 + (7 if turb else 5))),
+        # per cell, what the three directions share once: Q(5), V(1), T, Rmiu, Dst, Vol, DQ(18); Alagm(3),
+        # SD(9); GV(3 x 6) out
+        "k_visc_faces": ("cell", d * (5 + 1 + 1 + 1 + 1 + 1 + 18 + 3 + 9 + 18)),
+        # Q(3[,5]), V(1), PP, T, rad, shock once; Alagm(3), SD(9), Grad(3); G(3 x 5[,7]) out
+        "k_conv_faces": ("cell", d * ((6 if turb else 4) + 4 + 3 + 9 + 3 + 3 * (7 if turb else 5))),
         # ghost cells of the three layers beyond each face: V(1:4[,6:7]) in, Q(3[,5]) out
         "k_prim_ghost": ("ghost", d * ((6 if turb else 4) + (5 if turb else 3))),
         # per cell: G 3 x 7, GV 3 x 6 (viscous), V(1,3,4), Yc, Zc, Vol; D(7) out

@@ -126,35 +126,44 @@ __device__ __forceinline__ void decode3(int lin, int ni, int nj, int& i, int& j,
     k += 1;
 }
 
-// Faces of one block in FTA x FTB tiles of the plane spanned by i and the stencil direction
-// DIR (2: the (i, j) plane, then k; 3: the (i, k) plane, then j), 256 per workgroup: the
-// neighbours a face stencil reads along DIR are read by the same workgroup, so they come from
-// the L2 of one XCD instead of being fetched again by workgroups that the dispatcher put on
-// other XCDs, while each wave still reads one row of 64 consecutive i.  Returns false for the
-// padding of partial tiles.
-#ifndef TRANS_FTA
-#define TRANS_FTA 64
-#define TRANS_FTB 4
-#endif
-constexpr int FTA = TRANS_FTA, FTB = TRANS_FTB;
-template <int DIR>
-__device__ __forceinline__ bool decode_face_tile(int lin, int n0, int n1, int n2, int& i, int& j, int& k)
+// One workgroup's share of a block in bricks of rows j0 .. j0 + h - 1, all i and k: the 256
+// elements of the brick from `base` on, i fastest, then j, then k.  The elements are the cells, or
+// the points (i, j, k), 1..NI x 1..NJ x 1..NK, each of which stands for the faces on its low
+// sides.  blk < 0: padding.
+struct BrickSeg {
+    int blk, j0, h, base;
+};
+
+// The face kernels' grid: workgroup q does direction (q / 8) % 3 + 1 of table entry
+// q / 24 * 8 + q % 8.  Workgroups go round the eight XCDs, so the three directions of an entry run
+// beside each other on one XCD, and what they all read (gradients, primitives, geometry of the
+// same cells) comes from that XCD's L2 for two of the three.
+__device__ __forceinline__ int face_entry(int q, int& dir)
 {
-    const int tile = lin / (FTA * FTB), w = lin % (FTA * FTB);
-    const int ti = w % FTA, tm = w / FTA;
-    const int ntx = (n0 + FTA - 1) / FTA;
-    const int tx = tile % ntx;
-    i = tx * FTA + ti + 1;
-    if (DIR == 2) {
-        const int nty = (n1 + FTB - 1) / FTB;
-        j = (tile / ntx) % nty * FTB + tm + 1;
-        k = tile / (ntx * nty) + 1;
-        return i <= n0 && j <= n1;
-    }
-    const int ntz = (n2 + FTB - 1) / FTB;
-    k = (tile / ntx) % ntz * FTB + tm + 1;
-    j = tile / (ntx * ntz) + 1;
-    return i <= n0 && k <= n2;
+    dir = (q >> 3) % 3 + 1;
+    return q / 24 * 8 + (q & 7);
+}
+
+// The point of thread t, and whether it has a face of direction `dir`.
+__device__ __forceinline__ bool face_point(const BrickSeg& s, const BlkInfo& b, int t, int dir, int& i, int& j, int& k)
+{
+    const int lin = s.base + t;
+    i = lin % b.ni + 1;
+    const int r = lin / b.ni;
+    j = s.j0 + r % s.h;
+    k = r / s.h + 1;
+    return k <= b.nk && (dir == 1 || i < b.ni) && (dir == 2 || j < b.nj) && (dir == 3 || k < b.nk);
+}
+
+// The cell of thread t, and whether there is one.
+__device__ __forceinline__ bool brick_cell(const BrickSeg& s, const BlkInfo& b, int t, int& i, int& j, int& k)
+{
+    const int lin = s.base + t;
+    i = lin % (b.ni - 1) + 1;
+    const int r = lin / (b.ni - 1);
+    j = s.j0 + r % s.h;
+    k = r / s.h + 1;
+    return k < b.nk;
 }
 
 // Hyperplane-major index of interior cell (i,j,k) for the line-march sweeps.  Lines run

@@ -143,15 +143,13 @@ __device__ __forceinline__ CellQ face_q(const Fields& f, int d, long cm, long cp
 template <bool FSCHEME>
 __global__ void __launch_bounds__(256) k_gradients(trans_params p, int if_turb, Fields f,
                                                    const BlkInfo* __restrict__ blks,
-                                                   const Seg* __restrict__ seg)
+                                                   const BrickSeg* __restrict__ seg)
 {
-    const Seg s = seg[blockIdx.x];
+    const BrickSeg s = seg[blockIdx.x];
+    if (s.blk < 0) return;
     const BlkInfo b = blks[s.blk];
-    const int NI1 = b.ni - 1, NJ1 = b.nj - 1, NK1 = b.nk - 1;
-    const int lin = s.base + threadIdx.x;
-    if (lin >= NI1 * NJ1 * NK1) return;
     int i, j, k;
-    decode3(lin, NI1, NJ1, i, j, k);
+    if (!brick_cell(s, b, threadIdx.x, i, j, k)) return;
     const long c = cidx(b, i, j, k);
     const long tot = f.tot;
     const bool turb = if_turb != 0;
@@ -390,35 +388,45 @@ __device__ __forceinline__ void visc_face_flux(const trans_params& p, bool turb,
     out[5] = (vmuoq * (go[0] * Dx + go[1] * Dy + go[2] * Dz)) / p.ref;
 }
 
-// One thread per face of direction DIR: GV[DIR-1] receives visc_face_flux.
 template <int DIR>
-__global__ void __launch_bounds__(256, 3) k_visc_face(trans_params p, int if_turb, Fields f,
-                                                   const BlkInfo* __restrict__ blks,
-                                                   const Seg* __restrict__ seg)
+__device__ __forceinline__ void visc_face_store(const trans_params& p, bool turb, const Fields& f, const BlkInfo& b,
+                                                int i, int j, int k)
 {
-    const Seg s = seg[blockIdx.x];
-    const BlkInfo b = blks[s.blk];
-    const int n0 = DIR == 1 ? b.ni : b.ni - 1;
-    const int n1 = DIR == 2 ? b.nj : b.nj - 1;
-    const int n2 = DIR == 3 ? b.nk : b.nk - 1;
-    const int lin = s.base + threadIdx.x;
-    int i, j, k;
-    if (DIR == 1) {
-        if (lin >= n0 * n1 * n2) return;
-        decode3(lin, n0, n1, i, j, k);
-    } else if (!decode_face_tile<DIR>(lin, n0, n1, n2, i, j, k)) {
-        return;
-    }
     double o[6];
-    visc_face_flux<DIR>(p, if_turb != 0, f, b, i, j, k, o);
+    visc_face_flux<DIR>(p, turb, f, b, i, j, k, o);
     const long c0 = cidx(b, i, j, k), tot = f.tot;
     double* G = f.GV[DIR - 1];
 #pragma unroll
     for (int q = 0; q < 4; q++) G[(long)q * tot + c0] = o[q];
-    if (if_turb) {
+    if (turb) {
         G[4 * tot + c0] = o[4];
         G[5 * tot + c0] = o[5];
     }
+}
+
+// One thread per face, all three directions in one launch: GV[DIR-1] receives visc_face_flux.
+// Bound by instruction issue and the latency of a wave's loads (three waves per SIMD at 161
+// registers; at four it spills): 1483 vector instructions and 81 loads per face, 4.9 GB at 8.1M
+// cells.  As three launches, one per direction, it read 8.5 GB, since each read the gradients and
+// primitives from memory: 2114 us then, 1895 us now; at 0.13M cells, where the three ran on three
+// streams that had to be forked and joined, 91 us of kernels then, 43 us now.  One thread for a
+// cell's three faces takes 1990 us.
+__global__ void __launch_bounds__(256, 3) k_visc_faces(trans_params p, int if_turb, Fields f,
+                                                    const BlkInfo* __restrict__ blks,
+                                                    const BrickSeg* __restrict__ seg)
+{
+    int dir, i, j, k;
+    const BrickSeg s = seg[face_entry(blockIdx.x, dir)];
+    if (s.blk < 0) return;
+    const BlkInfo b = blks[s.blk];
+    if (!face_point(s, b, threadIdx.x, dir, i, j, k)) return;
+    const bool turb = if_turb != 0;
+    if (dir == 1)
+        visc_face_store<1>(p, turb, f, b, i, j, k);
+    else if (dir == 2)
+        visc_face_store<2>(p, turb, f, b, i, j, k);
+    else
+        visc_face_store<3>(p, turb, f, b, i, j, k);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -661,35 +669,42 @@ __device__ __forceinline__ void conv_face_flux(const trans_params& p, bool turb,
     out[6] = dTO;
 }
 
-// One thread per face of direction DIR: G[DIR-1] receives conv_face_flux.
 template <int DIR, int SPATIAL, int ROE>
-__global__ void __launch_bounds__(256) k_conv_face(trans_params p, int if_turb, Fields f,
-                                                   const BlkInfo* __restrict__ blks,
-                                                   const Seg* __restrict__ seg)
+__device__ __forceinline__ void conv_face_store(const trans_params& p, bool turb, const Fields& f, const BlkInfo& b,
+                                                int i, int j, int k)
 {
-    const Seg s = seg[blockIdx.x];
-    const BlkInfo b = blks[s.blk];
-    const int n0 = DIR == 1 ? b.ni : b.ni - 1;
-    const int n1 = DIR == 2 ? b.nj : b.nj - 1;
-    const int n2 = DIR == 3 ? b.nk : b.nk - 1;
-    const int lin = s.base + threadIdx.x;
-    int i, j, k;
-    if (DIR == 1) {
-        if (lin >= n0 * n1 * n2) return;
-        decode3(lin, n0, n1, i, j, k);
-    } else if (!decode_face_tile<DIR>(lin, n0, n1, n2, i, j, k)) {
-        return;
-    }
     double o[7];
-    conv_face_flux<DIR, SPATIAL, ROE>(p, if_turb != 0, f, b, i, j, k, o);
+    conv_face_flux<DIR, SPATIAL, ROE>(p, turb, f, b, i, j, k, o);
     const long c0 = cidx(b, i, j, k), tot = f.tot;
     double* G = f.G[DIR - 1];
 #pragma unroll
     for (int L = 0; L < 5; L++) G[(long)L * tot + c0] = o[L];
-    if (if_turb) {
+    if (turb) {
         G[5 * tot + c0] = o[5];
         G[6 * tot + c0] = o[6];
     }
+}
+
+// One thread per face, all three directions in one launch: G[DIR-1] receives conv_face_flux.
+// Bound by instruction issue: 70 % of the vector cycles at 8.1M cells (MUSCL + Roe), 1186 us as
+// three launches, 1155 us as one; at 0.13M cells 65 us then, 30 us now.
+template <int SPATIAL, int ROE>
+__global__ void __launch_bounds__(256) k_conv_faces(trans_params p, int if_turb, Fields f,
+                                                    const BlkInfo* __restrict__ blks,
+                                                    const BrickSeg* __restrict__ seg)
+{
+    int dir, i, j, k;
+    const BrickSeg s = seg[face_entry(blockIdx.x, dir)];
+    if (s.blk < 0) return;
+    const BlkInfo b = blks[s.blk];
+    if (!face_point(s, b, threadIdx.x, dir, i, j, k)) return;
+    const bool turb = if_turb != 0;
+    if (dir == 1)
+        conv_face_store<1, SPATIAL, ROE>(p, turb, f, b, i, j, k);
+    else if (dir == 2)
+        conv_face_store<2, SPATIAL, ROE>(p, turb, f, b, i, j, k);
+    else
+        conv_face_store<3, SPATIAL, ROE>(p, turb, f, b, i, j, k);
 }
 
 // ---------------------------------------------------------------------------------------
