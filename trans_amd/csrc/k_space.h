@@ -9,7 +9,11 @@
 // IF_Local_Sub = 1 (Input/ReadOrg.F90:155-156).  With preconditioning (:91-120) the acoustic
 // part of each direction uses the preconditioned speed sqrt(alf^2 |u|^2 + ub c^2) and the
 // convective part |u.S| (1 - alf), ub raised to that direction's viscous limit.
-__global__ void __launch_bounds__(256) k_spectral_radius(trans_params p, int ki, Fields f,
+// PRIM: also Q of the cell, as k_prim_cells forms it, for a residual that follows at once.  Bound by
+// memory (5 TB/s); the primitives cost 2 us beside it at 0.13M cells and 90 us at 8.1M, as a pass
+// of their own 7 us and 150 us.
+template <bool PRIM>
+__global__ void __launch_bounds__(256) k_spectral_radius(trans_params p, int ki, int if_turb, Fields f,
                                                          const BlkInfo* __restrict__ blks,
                                                          const Seg* __restrict__ seg)
 {
@@ -27,6 +31,15 @@ __global__ void __launch_bounds__(256) k_spectral_radius(trans_params p, int ki,
     const double Vxi = f.V[tot + c] / Den;
     const double Vyi = f.V[2 * tot + c] / Den;
     const double Vzi = f.V[3 * tot + c] / Den;
+    if (PRIM) {
+        f.Q[c] = Vxi;
+        f.Q[tot + c] = Vyi;
+        f.Q[2 * tot + c] = Vzi;
+        if (if_turb) {
+            f.Q[3 * tot + c] = f.V[5 * tot + c] / Den;
+            f.Q[4 * tot + c] = f.V[6 * tot + c] / Den;
+        }
+    }
     const double AAc = sqrt(1.4 * f.PP[c] / Den);
     const double RmiuL = sutherland(p, f.T[c]);
     const double RmiuTL = f.Rmiu[c];

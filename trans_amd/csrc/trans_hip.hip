@@ -1079,8 +1079,8 @@ static int launch_check(trans_ctx* c, const char* what)
 int trans_hip_spectral_radius(trans_ctx* c)
 {
     if (!c) return TRANS_EINVAL;
-    KLAUNCH(c, "k_spectral_radius", k_spectral_radius, dim3(c->seg_cell.n), dim3(WG), c->p, c->ki, c->f,
-                       c->d_blk, c->seg_cell.d);
+    KLAUNCH(c, "k_spectral_radius", k_spectral_radius<false>, dim3(c->seg_cell.n), dim3(WG), c->p, c->ki,
+            if_turb_now(c), c->f, c->d_blk, c->seg_cell.d);
     return launch_check(c, "k_spectral_radius");
 }
 
@@ -1151,17 +1151,18 @@ static bool launch_fused(trans_ctx* c, int if_turb)
 
 extern "C" {
 
-int trans_hip_space(trans_ctx* c)
+// prim: whether Q of the interior cells still has to be formed
+static int space_async(trans_ctx* c, bool prim)
 {
-    if (!c) return TRANS_EINVAL;
     const int if_turb = if_turb_now(c);
     const bool visc = c->p.if_euler == 0;
     const int nblk = (int)c->hb.size();
     int rc;
     // Q (u, v, w, k/rho, omega/rho) of every cell the gradient and face stencils read, formed
     // once: k_prim_cells for the interior cells, k_prim_ghost for the ghost layers
-    KLAUNCH(c, "k_prim_cells", k_prim_cells, dim3(c->seg_cell.n), dim3(WG), if_turb, c->f, c->d_blk,
-            c->seg_cell.d);
+    if (prim)
+        KLAUNCH(c, "k_prim_cells", k_prim_cells, dim3(c->seg_cell.n), dim3(WG), if_turb, c->f, c->d_blk,
+                c->seg_cell.d);
     KLAUNCH(c, "k_prim_ghost", k_prim_ghost, dim3(c->seg_ghost.n), dim3(WG), if_turb, c->f, c->d_blk,
             c->seg_ghost.d);
     if (visc) {
@@ -1184,6 +1185,12 @@ int trans_hip_space(trans_ctx* c)
     return launch_check(c, "space");
 }
 
+int trans_hip_space(trans_ctx* c)
+{
+    if (!c) return TRANS_EINVAL;
+    return space_async(c, true);
+}
+
 int trans_hip_residual(trans_ctx* c)
 {
     int rc;
@@ -1195,14 +1202,15 @@ int trans_hip_residual(trans_ctx* c)
         KLAUNCH_ON(c, c->aux[0], "k_bc_outlet", k_bc_outlet, dim3(c->n_outl), dim3(256), c->p, if_turb_now(c), c->f,
                    c->d_blk, c->d_patch, c->d_outl);
     }
-    if ((rc = trans_hip_spectral_radius(c))) return rc;
+    KLAUNCH(c, "k_spectral_radius", k_spectral_radius<true>, dim3(c->seg_cell.n), dim3(WG), c->p, c->ki,
+            if_turb_now(c), c->f, c->d_blk, c->seg_cell.d);
+    if ((rc = launch_check(c, "k_spectral_radius"))) return rc;
     if (c->n_bcseg)
         KLAUNCH(c, "k_bc", k_bc, dim3(c->n_bcseg), dim3(128), c->p, if_turb_now(c), -1, c->f, c->d_blk, c->d_patch,
                 c->d_bcseg);
     if (outl) join_aux(c, 1);
     if ((rc = launch_check(c, "k_bc"))) return rc;
-    if ((rc = trans_hip_space(c))) return rc;
-    return 0;
+    return space_async(c, false);
 }
 
 }  // extern "C"
@@ -1557,8 +1565,8 @@ static int plain_body(trans_ctx* c)
     auto cells = [&](const SegTable& t, int b) { return dim3(t.wrange[b + 1] - t.wrange[b]); };
     for (int s = 0; s < nsub; s++) {
         for (int b = 0; b < nblk; b++)
-            KLAUNCH(c, "k_spectral_radius", k_spectral_radius, cells(c->seg_cell, b), dim3(WG), c->p, c->ki, c->f,
-                    c->d_blk, c->seg_cell.d + c->seg_cell.wrange[b]);
+            KLAUNCH(c, "k_spectral_radius", k_spectral_radius<false>, cells(c->seg_cell, b), dim3(WG), c->p, c->ki,
+                    if_turb, c->f, c->d_blk, c->seg_cell.d + c->seg_cell.wrange[b]);
         for (int b = 0; b < nblk; b++) {
             if (c->bc_wrange[b + 1] > c->bc_wrange[b])
                 KLAUNCH(c, "k_bc", k_bc, dim3(c->bc_wrange[b + 1] - c->bc_wrange[b]), dim3(128), c->p, if_turb, -1, c->f,
