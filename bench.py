@@ -72,6 +72,9 @@ def alg_bytes(name, neq, fp32, dual_shift=True):
         "k_wave_rhs": ("cell", d * (5 + 5 + 5 + 5 + 3 + 1 + 1 + (2 + 2 + 4 + 15 + 1 + 1 + 1 if turb else 0))
                        + r * (5 + 2 + 1 + 3 + 3 + (5 if turb else 0))),
         "k_wave_unskew": ("cell", (r + d) * neq),
+        # k_update_v with the increments from the packets, also written to D
+        "k_wave_update": ("cell", (r + d) * neq
+                          + d * (7 + 1 + 1 + 9 + 1 + 7 + 1 + 1 + 1 + (35 if dual_shift else 0))),
         # D(5), V(5), Wt0(5), Wt1(5), Rds(3), Dtm, Vol in; 17 sweep inputs out in the operator's precision
         "k_lusgs_rhs_w": ("cell", d * (5 + 5 + 5 + 5 + 3 + 1 + 1) + r * 17),
         "k_sst_rhs_w": ("cell", d * (2 + 3 + 2 + 2 + 15 + 1 + 1 + 1 + 1 + 3 + 1) + r * 3),

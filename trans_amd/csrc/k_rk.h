@@ -143,7 +143,7 @@ __global__ void __launch_bounds__(256) k_rk_update_v(trans_params p, int ki, int
             const double PPP = 0.4 * v5 - 0.2 * (sqr(v2) + sqr(v3) + sqr(v4)) / v1;
             const double TT = p.rxm2 * PPP / v1;
             const double RmiuL = (1.0 + p.csthlnd) / (TT + p.csthlnd) * pow(TT, 1.5);
-            sst_kw_update(p, f, c, v1, RmiuL);
+            sst_kw_update(p, f, c, f.D[5 * tot + c], f.D[6 * tot + c], v1, RmiuL);
         }
         dr[1] = fabs(f.D[5 * tot + c] / v1);
         dr[2] = fabs(f.D[6 * tot + c] / v1);

@@ -841,14 +841,13 @@ __device__ __forceinline__ void norm_combine(double& s, double& m, int& a, doubl
 }
 
 // k/omega update with positivity damping and the SST (or WD+) limiter on eddy viscosity
-// (Time/TIME_Update_V.F90:709-858, Time/TIME_RK_V_Update_New.F90:104-230): increments from
-// D(6:7), new k, omega and Rmiu written back.  pRo is the updated density and RmiuL the
+// (Time/TIME_Update_V.F90:709-858, Time/TIME_RK_V_Update_New.F90:104-230): increments AinRTk and
+// AinRTO, new k, omega and Rmiu written back.  pRo is the updated density and RmiuL the
 // laminar viscosity, which the two callers evaluate in their own forms.
-__device__ __forceinline__ void sst_kw_update(const trans_params& p, const Fields& f, long c, double pRo,
-                                              double RmiuL)
+__device__ __forceinline__ void sst_kw_update(const trans_params& p, const Fields& f, long c, double AinRTk,
+                                              double AinRTO, double pRo, double RmiuL)
 {
     const long tot = f.tot;
-    const double AinRTk = f.D[5 * tot + c], AinRTO = f.D[6 * tot + c];
     double ARTk = f.V[5 * tot + c], ARTO = f.V[6 * tot + c];
     if (AinRTk >= 0.0)
         ARTk = ARTk + AinRTk;
@@ -950,8 +949,94 @@ __device__ __forceinline__ void norm_reduce(const double dr[3], int arg, NormPar
     }
 }
 
+// One cell's update with the increments d (mean flow, k-omega) and its norms' terms.
 // shift: 0, or the Kind_Dual of a fused dual-time history shift (TIME_Update_U, as
 // k_update_u) of the updated state, for the last sub-iteration of an outer iteration.
+__device__ __forceinline__ void update_cell(const trans_params& p, int ki, int if_turb, const Fields& f, long c,
+                                            const double d[7], int shift, double dr[3])
+{
+    const long tot = f.tot;
+    const double v1 = f.V[c];
+    dr[0] = fabs(d[0] / v1);
+    dr[1] = fabs(d[5] / v1);
+    dr[2] = fabs(d[6] / v1);
+
+    const double AinRo = d[0], AinRx = d[1], AinRy = d[2], AinRz = d[3], AinRe = d[4];
+    double pRo = v1;
+    const double roinv = 1.0 / pRo;
+    const double rad = f.rad[c];
+    double vn[5];
+    if (p.if_precondition) {
+        // Time/TIME_Update_V.F90:522-606: the increment added to the conservative state; the
+        // kinetic energy divides by the density before the update, and T is formed from the
+        // pressure before the update
+        const double pRx = f.V[tot + c] + AinRx, pRy = f.V[2 * tot + c] + AinRy, pRz = f.V[3 * tot + c] + AinRz;
+        double pRe = fabs(f.V[4 * tot + c] + AinRe);
+        pRo = fabs(pRo + AinRo);
+        const double DV = 0.5 * (pRx * pRx + pRy * pRy + pRz * pRz) * roinv;
+        double pPP = (pRe - DV) * (1.4 - 1.0);
+        if (pPP <= 0.0) {
+            pPP = fabs(pPP);
+            pRe = pPP / (1.4 - 1.0) + DV;
+        }
+        f.T[c] = p.rxm2 * f.PP[c] / pRo;
+        f.PP[c] = pPP;
+        vn[0] = pRo;
+        vn[1] = pRx;
+        vn[2] = pRy;
+        vn[3] = pRz;
+        vn[4] = pRe;
+    } else {
+        double pVx = f.V[tot + c] * roinv;
+        double pVy = f.V[2 * tot + c] * roinv;
+        double pVz = f.V[3 * tot + c] * roinv;
+        const double AinX = (AinRx - pVx * AinRo) * roinv;
+        const double AinY = (AinRy - pVy * AinRo) * roinv;
+        const double AinZ = (AinRz - pVz * AinRo) * roinv;
+        const double AinP = (1.4 - 1.0) * (AinRe - 0.5 * AinRo * (pVx * pVx + pVy * pVy + pVz * pVz) -
+                                           pRo * (AinX * pVx + AinY * pVy + AinZ * pVz));
+        if (AinRo >= 0.)
+            pRo = pRo + AinRo;
+        else
+            pRo = pRo * exp(AinRo / (pRo + 1.e-10));
+        pRo = fabs(pRo);
+        double pp = f.PP[c];
+        if (AinP >= 0.)
+            pp = pp + AinP;
+        else
+            pp = pp * exp(AinP / (pp + 1.e-10));
+        pp = fabs(pp);
+        f.PP[c] = pp;
+        f.T[c] = p.rxm2 * pp / pRo;
+        pVx = pVx + AinX;
+        pVy = pVy + AinY;
+        pVz = pVz + AinZ;
+        const double DV = 0.5 * (pVx * pVx + pVy * pVy + pVz * pVz);
+        vn[0] = pRo;
+        vn[1] = pRo * pVx;
+        vn[2] = pRo * pVy;
+        vn[3] = pRo * pVz;
+        vn[4] = pp / (1.4 - 1.0) + DV * pRo - 0.5 * sqr(p.omega1 * rad) * pRo;
+    }
+#pragma unroll
+    for (int L = 0; L < 5; L++) f.V[(long)L * tot + c] = vn[L];
+
+    if (p.if_euler == 0 && if_turb == 1 && ki >= p.kitm) {
+        const double VV = sqr(vn[1]) + sqr(vn[2]) + sqr(vn[3]);
+        const double PPP = (1.4 - 1.0) * vn[4] - 0.5 * (1.4 - 1.0) * (VV / pRo - sqr(p.omega1 * rad) * pRo);
+        const double TT = p.rxm2 * PPP / pRo;
+        sst_kw_update(p, f, c, d[5], d[6], pRo, sutherland(p, TT));
+    }
+    if (shift) {
+#pragma unroll
+        for (int L = 0; L < TRANS_ML; L++) {
+            const long e = (long)L * tot + c;
+            if (shift == 2) f.Wt1[e] = f.Wt0[e];
+            f.Wt0[e] = f.V[e];
+        }
+    }
+}
+
 __global__ void __launch_bounds__(256) k_update_v(trans_params p, int ki, int if_turb, Fields f,
                                                   const BlkInfo* __restrict__ blks,
                                                   const Seg* __restrict__ seg, NormPart* part, int shift)
@@ -960,7 +1045,6 @@ __global__ void __launch_bounds__(256) k_update_v(trans_params p, int ki, int if
     const BlkInfo b = blks[s.blk];
     const int NI1 = b.ni - 1, NJ1 = b.nj - 1, NK1 = b.nk - 1;
     const int lin = s.base + threadIdx.x;
-    const long tot = f.tot;
     double dr[3] = {0.0, 0.0, 0.0};
     int arg = -1;
     if (lin < NI1 * NJ1 * NK1) {
@@ -968,86 +1052,10 @@ __global__ void __launch_bounds__(256) k_update_v(trans_params p, int ki, int if
         decode3(lin, NI1, NJ1, i, j, k);
         arg = lin;
         const long c = cidx(b, i, j, k);
-        const double v1 = f.V[c];
-        dr[0] = fabs(f.D[c] / v1);
-        dr[1] = fabs(f.D[5 * tot + c] / v1);
-        dr[2] = fabs(f.D[6 * tot + c] / v1);
-
-        const double AinRo = f.D[c], AinRx = f.D[tot + c], AinRy = f.D[2 * tot + c];
-        const double AinRz = f.D[3 * tot + c], AinRe = f.D[4 * tot + c];
-        double pRo = v1;
-        const double roinv = 1.0 / pRo;
-        const double rad = f.rad[c];
-        double vn[5];
-        if (p.if_precondition) {
-            // Time/TIME_Update_V.F90:522-606: the increment added to the conservative state; the
-            // kinetic energy divides by the density before the update, and T is formed from the
-            // pressure before the update
-            const double pRx = f.V[tot + c] + AinRx, pRy = f.V[2 * tot + c] + AinRy, pRz = f.V[3 * tot + c] + AinRz;
-            double pRe = fabs(f.V[4 * tot + c] + AinRe);
-            pRo = fabs(pRo + AinRo);
-            const double DV = 0.5 * (pRx * pRx + pRy * pRy + pRz * pRz) * roinv;
-            double pPP = (pRe - DV) * (1.4 - 1.0);
-            if (pPP <= 0.0) {
-                pPP = fabs(pPP);
-                pRe = pPP / (1.4 - 1.0) + DV;
-            }
-            f.T[c] = p.rxm2 * f.PP[c] / pRo;
-            f.PP[c] = pPP;
-            vn[0] = pRo;
-            vn[1] = pRx;
-            vn[2] = pRy;
-            vn[3] = pRz;
-            vn[4] = pRe;
-        } else {
-            double pVx = f.V[tot + c] * roinv;
-            double pVy = f.V[2 * tot + c] * roinv;
-            double pVz = f.V[3 * tot + c] * roinv;
-            const double AinX = (AinRx - pVx * AinRo) * roinv;
-            const double AinY = (AinRy - pVy * AinRo) * roinv;
-            const double AinZ = (AinRz - pVz * AinRo) * roinv;
-            const double AinP = (1.4 - 1.0) * (AinRe - 0.5 * AinRo * (pVx * pVx + pVy * pVy + pVz * pVz) -
-                                               pRo * (AinX * pVx + AinY * pVy + AinZ * pVz));
-            if (AinRo >= 0.)
-                pRo = pRo + AinRo;
-            else
-                pRo = pRo * exp(AinRo / (pRo + 1.e-10));
-            pRo = fabs(pRo);
-            double pp = f.PP[c];
-            if (AinP >= 0.)
-                pp = pp + AinP;
-            else
-                pp = pp * exp(AinP / (pp + 1.e-10));
-            pp = fabs(pp);
-            f.PP[c] = pp;
-            f.T[c] = p.rxm2 * pp / pRo;
-            pVx = pVx + AinX;
-            pVy = pVy + AinY;
-            pVz = pVz + AinZ;
-            const double DV = 0.5 * (pVx * pVx + pVy * pVy + pVz * pVz);
-            vn[0] = pRo;
-            vn[1] = pRo * pVx;
-            vn[2] = pRo * pVy;
-            vn[3] = pRo * pVz;
-            vn[4] = pp / (1.4 - 1.0) + DV * pRo - 0.5 * sqr(p.omega1 * rad) * pRo;
-        }
+        double d[7];
 #pragma unroll
-        for (int L = 0; L < 5; L++) f.V[(long)L * tot + c] = vn[L];
-
-        if (p.if_euler == 0 && if_turb == 1 && ki >= p.kitm) {
-            const double VV = sqr(vn[1]) + sqr(vn[2]) + sqr(vn[3]);
-            const double PPP = (1.4 - 1.0) * vn[4] - 0.5 * (1.4 - 1.0) * (VV / pRo - sqr(p.omega1 * rad) * pRo);
-            const double TT = p.rxm2 * PPP / pRo;
-            sst_kw_update(p, f, c, pRo, sutherland(p, TT));
-        }
-        if (shift) {
-#pragma unroll
-            for (int L = 0; L < TRANS_ML; L++) {
-                const long e = (long)L * tot + c;
-                if (shift == 2) f.Wt1[e] = f.Wt0[e];
-                f.Wt0[e] = f.V[e];
-            }
-        }
+        for (int L = 0; L < 7; L++) d[L] = f.D[(long)L * f.tot + c];
+        update_cell(p, ki, if_turb, f, c, d, shift, dr);
     }
     norm_reduce(dr, arg, part, 0);
 }

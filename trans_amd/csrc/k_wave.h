@@ -221,14 +221,18 @@ __global__ void __launch_bounds__(256) k_wave_rhs(trans_params p, Fields f, cons
     }
 }
 
-// Increments D(c0+1..c0+neq) from the packets back to D, tile by tile through LDS.
-template <typename R>
-__global__ void __launch_bounds__(256) k_wave_unskew(int c0, int neq, Fields f, const BlkInfo* __restrict__ blks,
-                                                     const Seg* __restrict__ seg)
+// NEQ increments (7: mean flow and k-omega, 5, or 2: k-omega) of a tile of cells from the packets into
+// LDS, diagonal by diagonal: sv[L][tj * WT + ti] for L = 5 (NEQ 2) or 0 on.
+template <typename R, int NEQ>
+__device__ __forceinline__ void wave_fetch(const Fields& f, const Seg& s, const BlkInfo& b, R (*sv)[WT * WT])
 {
-    __shared__ R sv[7][WT * WT];
-    const Seg s = seg[blockIdx.x];
-    const BlkInfo b = blks[s.blk];
+    constexpr int VL = WaveRow<R>::VL;
+    struct alignas(16) Vec {
+        R x[VL];
+    };
+    struct alignas(2 * sizeof(R)) Two {
+        R x[2];
+    };
     for (int q = threadIdx.x; q < (2 * WT - 1) * WT; q += 256) {
         const int ti = q % WT, tj = q / WT - ti;
         if (tj < 0 || tj >= WT) continue;
@@ -236,14 +240,72 @@ __global__ void __launch_bounds__(256) k_wave_unskew(int c0, int neq, Fields f, 
         if (!ic.ok) continue;
         int lane;
         const R* const row = (const R*)f.P + wave_row<R>(b, ic.i, ic.j, ic.k, lane);
-        for (int L = c0; L < c0 + neq; L++)
-            sv[L][tj * WT + ti] = row[wave_elem<R>(L < 5 ? WV_D + L : WV_K + L - 5, lane)];
+        const int o = tj * WT + ti;
+        if (NEQ != 2) {
+#pragma unroll
+            for (int v = WV_D; v < WV_D + 4; v += VL) {
+                const Vec x = *reinterpret_cast<const Vec*>(row + wave_elem<R>(v, lane));
+#pragma unroll
+                for (int e = 0; e < VL; e++) sv[v - WV_D + e][o] = x.x[e];
+            }
+            sv[4][o] = row[wave_elem<R>(WV_D + 4, lane)];
+        }
+        if (NEQ != 5) {
+            const Two x = *reinterpret_cast<const Two*>(row + wave_elem<R>(WV_K, lane));
+            sv[5][o] = x.x[0];
+            sv[6][o] = x.x[1];
+        }
     }
     __syncthreads();
+}
+
+// The k-omega increments back to D (the Runge-Kutta path), tile by tile.
+template <typename R>
+__global__ void __launch_bounds__(256) k_wave_unskew(Fields f, const BlkInfo* __restrict__ blks,
+                                                     const Seg* __restrict__ seg)
+{
+    __shared__ R sv[7][WT * WT];
+    const Seg s = seg[blockIdx.x];
+    const BlkInfo b = blks[s.blk];
+    wave_fetch<R, 2>(f, s, b, sv);
     const TileCell oc = wtile_cell(s, b, threadIdx.x % WT, threadIdx.x / WT);
     if (!oc.ok) return;
     const long c = cidx(b, oc.i, oc.j, oc.k);
-    for (int L = c0; L < c0 + neq; L++) f.D[(long)L * f.tot + c] = (double)sv[L][threadIdx.x];
+    for (int L = 5; L < 7; L++) f.D[(long)L * f.tot + c] = (double)sv[L][threadIdx.x];
+}
+
+// k_update_v with the increments from the packets, which go to D as well: a workgroup updates a
+// WT x WT tile of cells.  Bound by memory (4.8 TB/s at 8.1M cells): 858 us, with a pass of its own for
+// the increments 777 + 231 us; 0.13M cells, 24 us and 33 us.
+template <typename R, int NEQ>
+__global__ void __launch_bounds__(256) k_wave_update(trans_params p, int ki, int if_turb, Fields f,
+                                                     const BlkInfo* __restrict__ blks, const Seg* __restrict__ seg,
+                                                     NormPart* part, int shift)
+{
+    __shared__ R sv[7][WT * WT];
+    const Seg s = seg[blockIdx.x];
+    const BlkInfo b = blks[s.blk];
+    wave_fetch<R, NEQ>(f, s, b, sv);
+    const TileCell oc = wtile_cell(s, b, threadIdx.x % WT, threadIdx.x / WT);
+    double dr[3] = {0.0, 0.0, 0.0};
+    int arg = -1;
+    if (oc.ok) {
+        const long c = cidx(b, oc.i, oc.j, oc.k);
+        arg = oc.i - 1 + (b.ni - 1) * (oc.j - 1 + (b.nj - 1) * (oc.k - 1));
+        double d[7];
+#pragma unroll
+        for (int L = 0; L < 7; L++) {
+            double* const D = f.D + (long)L * f.tot + c;
+            if (L < NEQ) {
+                d[L] = (double)sv[L][threadIdx.x];
+                *D = d[L];
+            } else {
+                d[L] = *D;
+            }
+        }
+        update_cell(p, ki, if_turb, f, c, d, shift, dr);
+    }
+    norm_reduce(dr, arg, part, 0);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -523,10 +585,13 @@ __device__ __forceinline__ void wave_sweep(const Fields& f, const BlkInfo& b, in
                 else
                     dq[L] = FORWARD ? wv_fma(x.d[L], x.sa, sum * x.sb) * x.rf1 : wv_fma(-(sum * x.sb), x.rf1, x.d[L]);
             }
-            if constexpr (!MF) return dq[0] + dq[1];
-            hu2 = R(0.5) * wv_dot<UF>(x.u, x.u);
-            e = wv_fma(hu2, dq[0], dq[4] - wv_dot<false>(x.u, dq + 1));
-            return e;
+            if constexpr (!MF) {
+                return dq[0] + dq[1];
+            } else {
+                hu2 = R(0.5) * wv_dot<UF>(x.u, x.u);
+                e = wv_fma(hu2, dq[0], dq[4] - wv_dot<false>(x.u, dq + 1));
+                return e;
+            }
         };
         R chk = front();
         if (__builtin_expect(__any(chk != chk), 0)) {
@@ -536,12 +601,12 @@ __device__ __forceinline__ void wave_sweep(const Fields& f, const BlkInfo& b, in
             for (int spins = 0;; spins++) {
                 // the next row's as well: a wave that follows its upstream tile that closely would
                 // otherwise poll on every row
-                bool pend = false;
+                int pend = 0;
 #pragma unroll
                 for (int r = 0; r < 2; r++) {
                     const WaveIn<R, NEQ>& y = ring[(Q + r) % PD];
 #pragma unroll
-                    for (int L = 0; L < NEQ; L++) pend |= wv_pending<R>(y.ea[L]) | wv_pending<R>(y.eb[L]);
+                    for (int L = 0; L < NEQ; L++) pend |= (int)wv_pending<R>(y.ea[L]) | (int)wv_pending<R>(y.eb[L]);
                 }
                 if (!__any(pend)) break;
                 if (spins > spin_limit ||

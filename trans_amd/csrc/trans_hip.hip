@@ -89,7 +89,8 @@ struct trans_ctx {
     SegTable seg_rtile;
     int rt_kchunk = 8;
     int fused = 0;
-    int* d_wrange = nullptr;
+    int* d_wrange = nullptr;  // per-block first workgroup of seg_cell; of seg_wtile
+    int* d_trange = nullptr;
     NormPart* d_part = nullptr;
     trans_resid* d_resid = nullptr;
     double* d_mon = nullptr;  // 6 doubles: result of k_plane_integrals
@@ -791,7 +792,9 @@ static int create_ctx(const trans_params* params, int nblk, const trans_block_de
     }
     if ((rc = dalloc(c, &c->d_wrange, nblk + 1))) return rc;
     if ((rc = h2d(c, c->d_wrange, c->seg_cell.wrange.data(), (nblk + 1) * sizeof(int)))) return rc;
-    if ((rc = dalloc(c, &c->d_part, c->seg_cell.n)) || (rc = dalloc(c, &c->d_resid, nblk)) ||
+    if ((rc = dalloc(c, &c->d_trange, nblk + 1))) return rc;
+    if ((rc = h2d(c, c->d_trange, c->seg_wtile.wrange.data(), (nblk + 1) * sizeof(int)))) return rc;
+    if ((rc = dalloc(c, &c->d_part, std::max(c->seg_cell.n, c->seg_wtile.n))) || (rc = dalloc(c, &c->d_resid, nblk)) ||
         (rc = dalloc(c, &c->d_mon, 6)) || (rc = dalloc(c, &c->d_err, 1)))
         return rc;
     if (!dry) HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1298,19 +1301,30 @@ static void launch_wave_rule(trans_ctx* c)
         launch_wave_sweeps<R, NEQ, ALT, 2, 4>(c);
 }
 
-// Packet inputs, both wave sweeps and the increments back to D for NEQ = 7, 5 or 2 equations.
+// Packet inputs and both wave sweeps for NEQ = 7, 5 or 2 equations, and with 2 the increments back to D
+// (with the mean flow the update takes them from the packets).
 template <typename R, int NEQ>
 static void launch_wave(trans_ctx* c)
 {
-    const bool kw = NEQ == 2;
     KLAUNCH(c, "k_wave_rhs", (k_wave_rhs<R, NEQ != 2, NEQ != 5>), dim3(c->seg_wtile.n), dim3(WG), c->p, c->f, c->d_blk,
             c->seg_wtile.d, c->d_tctr, (uint4*)c->wave_edge, (long)(2 * (size_t)c->edge_n * sizeof(R) / 16));
     if (c->wave_alt)
         launch_wave_rule<R, NEQ, true>(c);
     else
         launch_wave_rule<R, NEQ, false>(c);
-    KLAUNCH(c, "k_wave_unskew", k_wave_unskew<R>, dim3(c->seg_wtile.n), dim3(WG), kw ? 5 : 0, NEQ, c->f, c->d_blk,
-            c->seg_wtile.d);
+    if constexpr (NEQ == 2)
+        KLAUNCH(c, "k_wave_unskew", k_wave_unskew<R>, dim3(c->seg_wtile.n), dim3(WG), c->f, c->d_blk, c->seg_wtile.d);
+}
+
+// The wave sweeps and the update of the state.
+template <typename R, int NEQ>
+static void launch_wave_step(trans_ctx* c, int shift)
+{
+    launch_wave<R, NEQ>(c);
+    KLAUNCH(c, "k_wave_update", (k_wave_update<R, NEQ>), dim3(c->seg_wtile.n), dim3(WG), c->p, c->ki, if_turb_now(c),
+            c->f, c->d_blk, c->seg_wtile.d, c->d_part, shift);
+    KLAUNCH(c, "k_norm_final", k_norm_final, dim3((int)c->hb.size()), dim3(256), c->d_part, c->d_trange, c->d_blk,
+            c->d_resid);
 }
 
 extern "C" {
@@ -1325,14 +1339,16 @@ static int lusgs_update_async(trans_ctx* c, int shift = 0)
     const int neq = if_turb ? 7 : 5;
     if (c->wave) {
         if (c->p.implicit_fp32 && if_turb)
-            launch_wave<float, 7>(c);
+            launch_wave_step<float, 7>(c, shift);
         else if (c->p.implicit_fp32)
-            launch_wave<float, 5>(c);
+            launch_wave_step<float, 5>(c, shift);
         else if (if_turb)
-            launch_wave<double, 7>(c);
+            launch_wave_step<double, 7>(c, shift);
         else
-            launch_wave<double, 5>(c);
-    } else if (wtiled && c->f.Wf)
+            launch_wave_step<double, 5>(c, shift);
+        return launch_check(c, "lusgs_update");
+    }
+    if (wtiled && c->f.Wf)
         KLAUNCH(c, "k_lusgs_rhs_w", k_lusgs_rhs_w<float>, dim3(c->seg_wtile.n), dim3(WG), c->p, c->f, c->d_blk,
                 c->seg_wtile.d);
     else if (wtiled)
@@ -1340,16 +1356,14 @@ static int lusgs_update_async(trans_ctx* c, int shift = 0)
                 c->seg_wtile.d);
     else
         KLAUNCH(c, "k_lusgs_rhs", k_lusgs_rhs, dim3(c->seg_cell.n), dim3(WG), c->p, c->f, c->d_blk, c->seg_cell.d);
-    if (if_turb && !c->wave) {
+    if (if_turb) {
         if (wtiled)
             KLAUNCH(c, "k_sst_rhs_w", k_sst_rhs_w, dim3(c->seg_wtile.n), dim3(WG), c->p, c->f, c->d_blk,
                     c->seg_wtile.d);
         else
             KLAUNCH(c, "k_sst_rhs", k_sst_rhs, dim3(c->seg_cell.n), dim3(WG), c->p, c->f, c->d_blk, c->seg_cell.d);
     }
-    if (c->wave) {
-        // done: the increments are in D
-    } else if (c->f.W || c->f.Wf) {
+    if (c->f.W || c->f.Wf) {
         // sweeps on the hyperplane-major buffer, increments back to D after
         if (c->p.implicit_fp32) {
             if (if_turb)
