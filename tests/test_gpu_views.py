@@ -74,3 +74,24 @@ def test_view_boxes(lo, hi):
             _cut(want, ilo, ihi)[...] = _cut(new[nm], ilo, ihi, lo)
         assert np.array_equal(a, want), nm
     sv.close()
+
+
+@pytest.mark.parametrize("size", [(33, 17, 9), (97, 81, 33)])
+def test_state_through_pinned_pieces(size):
+    """A whole state there and back: one piece of the pinned buffers, and many over several host
+    threads with arrays that begin inside a piece."""
+    blocks, org, glob = cases.bump_channel(*size)
+    prm = solver.prepare_case(blocks, org, glob)
+    sv = Solver(blocks, prm, ki=1)
+    rng = np.random.Generator(np.random.PCG64(5))
+    names = ("v", "pp", "t", "rmiu", "wt0", "wt1", "wt2")
+    put = {nm: np.asfortranarray(rng.random(blocks[0][nm].shape)) for nm in names}
+    got = {nm: np.asfortranarray(np.zeros_like(a)) for nm, a in put.items()}
+    for arrays, call in ((put, sv.lib.trans_hip_set_state), (got, sv.lib.trans_hip_get_state)):
+        s = capi.TransStateView()
+        for nm, a in arrays.items():
+            setattr(s, nm, capi.fview(a))
+        assert call(sv.ctx, 0, C.byref(s)) == 0
+    for nm in names:
+        assert np.array_equal(put[nm], got[nm]), nm
+    sv.close()

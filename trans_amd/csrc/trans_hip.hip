@@ -26,6 +26,7 @@
 #include "k_visc.h"
 #include "k_wave.h"
 #include "k_view.h"
+#include "host_copy.h"
 
 namespace {
 
@@ -618,6 +619,7 @@ static int create_ctx(const trans_params* params, int nblk, const trans_block_de
 {
     if (!params || !blocks || !out || nblk <= 0) return TRANS_EINVAL;
     trans_ctx* c = new trans_ctx();
+    g_pins.attach();
     *out = c;
     c->dry = dry;
     int rc = check_params(c, params);
@@ -845,6 +847,7 @@ int trans_hip_destroy(trans_ctx* c)
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
+    g_pins.detach();
     return 0;
 }
 
@@ -884,10 +887,11 @@ struct ViewJob {
 // Moves the part of each view inside the block's device extent -2..N+2.  The boxes are repacked on
 // the device in the face-flux arrays, which hold nothing between a residual and the next, so an
 // array is one copy (an array too large for them, one per slab of k planes) instead of one per
-// component with a strided loop on the host.  Reading state and history of the 8.1M-cell sector in
-// 16 blocks (1.96 GB) took 458 ms, now 111 ms; of a 2k-cell block (1.6 MB) 361 us, now 196 us;
-// setting the state of a 0.2M-cell block (78 MB) 15.7 ms, now 2.7 ms.  The link to pageable host
-// memory bounds it (17 to 28 GB/s).
+// component with a strided loop on the host, and what lies side by side there moves in pieces
+// through pinned buffers (host_copy.h).  Reading state and history of the 8.1M-cell sector in 16
+// blocks (1.96 GB): 458 ms before, 111 ms with the runtime's copies, now 52 ms; of a 2k-cell block
+// (1.6 MB) 361, 196 and now 145 us; setting the state of a 0.2M-cell block (78 MB) 15.7, 2.7 and
+// now 2.2 ms.
 static int copy_views(trans_ctx* c, int blk, const ViewJob* jobs, int njobs, bool upload)
 {
     const HostBlock& h = c->hb[blk];
@@ -904,36 +908,40 @@ static int copy_views(trans_ctx* c, int blk, const ViewJob* jobs, int njobs, boo
     long used[3] = {0, 0, 0};
     std::vector<double> buf;
     auto flush = [&]() -> int {
-        for (Slab& s : slabs) {
-            const long n = (long)s.b.cells * s.b.ncomp;
+        // host buffers of the boxes that are no one range of their view
+        size_t nbuf = 0;
+        for (const Slab& s : slabs)
+            if (!s.dense) nbuf += (size_t)s.b.cells * s.b.ncomp;
+        buf.resize(nbuf);
+        std::vector<HostCopy> list;
+        double* next = buf.data();
+        auto rows = [&](const Slab& s, double* q, bool gather) {
             const long row = (long)s.b.n0 * s.b.ncomp;
             const int n2 = s.b.cells / (s.b.n0 * s.b.n1);
-            if (!s.dense) buf.resize((size_t)n);
-            double* const hp = s.dense ? s.host : buf.data();
-            auto rows = [&](bool gather) {
-                for (int k = 0; k < n2; k++)
-                    for (int j = 0; j < s.b.n1; j++) {
-                        double* const p = s.host + k * s.vplane + j * s.vrow;
-                        double* const q = buf.data() + (k * (long)s.b.n1 + j) * row;
-                        std::memcpy(gather ? q : p, gather ? p : q, (size_t)row * sizeof(double));
-                    }
-            };
-            if (upload) {
-                if (!s.dense) rows(true);
-                HIPCHK(c, hipMemcpyAsync(s.b.stage, hp, (size_t)n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-                if (!s.dense) HIPCHK(c, hipStreamSynchronize(c->stream));
+            for (int k = 0; k < n2; k++)
+                for (int j = 0; j < s.b.n1; j++, q += row) {
+                    double* const p = s.host + k * s.vplane + j * s.vrow;
+                    std::memcpy(gather ? q : p, gather ? p : q, (size_t)row * sizeof(double));
+                }
+        };
+        for (const Slab& s : slabs) {
+            const size_t n = (size_t)s.b.cells * s.b.ncomp;
+            if (!s.dense && upload) rows(s, next, true);
+            list.push_back(HostCopy{(char*)(s.dense ? s.host : next), (char*)s.b.stage, n * sizeof(double)});
+            if (!s.dense) next += n;
+        }
+        HIPCHK(c, host_copies(list, upload, c->stream));
+        for (size_t q = 0; q < slabs.size(); q++) {
+            const Slab& s = slabs[q];
+            if (upload)
                 hipLaunchKernelGGL(k_view<true>, dim3((s.b.cells + WG - 1) / WG), dim3(WG), 0, c->stream, s.b);
-            } else {
-                HIPCHK(c, hipMemcpyAsync(hp, s.b.stage, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-                if (s.dense) continue;
-                HIPCHK(c, hipStreamSynchronize(c->stream));
-                rows(false);
-            }
+            else if (!s.dense)
+                rows(s, (double*)list[q].host, false);
         }
         slabs.clear();
         used[0] = used[1] = used[2] = 0;
         HIPCHK(c, hipGetLastError());
-        HIPCHK(c, hipStreamSynchronize(c->stream));
+        if (upload) HIPCHK(c, hipStreamSynchronize(c->stream));
         return 0;
     };
     for (int q = 0; q < njobs; q++) {
