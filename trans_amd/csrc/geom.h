@@ -30,6 +30,41 @@ double* wd_scratch_for_current_device()
     }
     return wd_scratch_ptr[dev];
 }
+
+// Whether the sorted form of the wall distance pays.  It costs about 0.2 ms of sorting; every cell
+// against every panel takes at least 0.1 us per panel, the time of one workgroup: 20 000 cells and
+// 4 000 panels 664 us against 487 us sorted, 161 000 and 1 590 787 us against 867 us, 4 096 and 1 024
+// 264 us against 329 us.
+bool wb_worth(long ncell, long npanel)
+{
+    return npanel >= 2048 && ncell >= 4096 && ncell < (1L << 30) && npanel < (1L << 30);
+}
+
+// k_wb_* on stream s; behind dd (ncell) lies the memory of the sorted form.
+void launch_wb(hipStream_t s, const double* dc, long ncell, const double* dp, long npanel, double* dd)
+{
+    const int ntile = (int)((npanel + WB_TILE - 1) / WB_TILE);
+    char* m = (char*)(((size_t)(dd + ncell) + 127) / 128 * 128);
+    double4* sc = (double4*)m;
+    double4* sp = sc + ncell;
+    double* tb = (double*)(sp + npanel);
+    unsigned long long* box = (unsigned long long*)(tb + 6 * (long)ntile);
+    int* bins = (int*)(box + 12);
+    int* from = bins + 2 * WB_BINS;
+    hipLaunchKernelGGL(k_wb_clear, dim3(64), dim3(256), 0, s, box, bins);
+    const auto grid = [](long n) { return dim3((unsigned)((n + 255) / 256)); };
+    hipLaunchKernelGGL(k_wb_box, dim3(256), dim3(256), 0, s, dc, ncell, box);
+    hipLaunchKernelGGL(k_wb_box, dim3(64), dim3(256), 0, s, dp, npanel, box + 6);
+    hipLaunchKernelGGL(k_wb_count, grid(ncell), dim3(256), 0, s, dc, ncell, box, bins);
+    hipLaunchKernelGGL(k_wb_count, grid(npanel), dim3(256), 0, s, dp, npanel, box + 6, bins + WB_BINS);
+    hipLaunchKernelGGL(k_wb_scan, dim3(2), dim3(1024), 0, s, bins);
+    hipLaunchKernelGGL(k_wb_scatter, grid(ncell), dim3(256), 0, s, dc, ncell, box, bins, sc, from);
+    hipLaunchKernelGGL(k_wb_scatter, grid(npanel), dim3(256), 0, s, dp, npanel, box + 6, bins + WB_BINS, sp,
+                       (int*)nullptr);
+    hipLaunchKernelGGL(k_wb_tiles, dim3((unsigned)ntile), dim3(64), 0, s, sp, (int)npanel, ntile, tb);
+    hipLaunchKernelGGL(k_wb_distance, dim3((unsigned)((ncell + 63) / 64)), dim3(64), 0, s, sc,
+                       from, ncell, sp, (int)npanel, tb, ntile, dd);
+}
 }  // namespace
 
 extern "C" {
@@ -76,29 +111,44 @@ int trans_geom_wall_distance(const double* cells, long ncell, const double* pane
         return 0;
     }
     hipStream_t s = nullptr;
-    double *dc = nullptr, *dp = nullptr, *dd = nullptr;
+    // the points, the squared minima, and for the sorted form the points in order and its tables
+    bool sorted = wb_worth(ncell, npanel);
+    const long ntile = (npanel + WB_TILE - 1) / WB_TILE;
+    const size_t plain = 8 * (size_t)(4 * ncell + 3 * npanel);
+    const size_t more = 32 * (size_t)(ncell + npanel) + 48 * (size_t)ntile + 4 * (size_t)ncell + 8 * 12 +
+                        2 * WB_BINS * sizeof(int) + 256;
+    char* mem = nullptr;
+    if (sorted && hipMalloc(&mem, plain + more) != hipSuccess) {
+        (void)hipGetLastError();
+        mem = nullptr;
+        sorted = false;
+    }
     int rc = 0;
     auto ok = [&](hipError_t e) {
         if (e != hipSuccess && !rc) rc = TRANS_EHIP;
         return e == hipSuccess;
     };
-    if (ok(hipStreamCreateWithFlags(&s, hipStreamNonBlocking)) && ok(hipMalloc(&dc, 3 * ncell * sizeof(double))) &&
-        ok(hipMalloc(&dp, 3 * npanel * sizeof(double))) && ok(hipMalloc(&dd, ncell * sizeof(double))) &&
-        ok(hipMemcpyAsync(dc, cells, 3 * ncell * sizeof(double), hipMemcpyHostToDevice, s)) &&
-        ok(hipMemcpyAsync(dp, panels, 3 * npanel * sizeof(double), hipMemcpyHostToDevice, s))) {
-        const long per = 256L * WD_CPT;
-        hipLaunchKernelGGL(k_wall_distance, dim3((unsigned)((ncell + per - 1) / per)), dim3(256), 0, s, dc, ncell, dp,
-                           npanel, dd);
-        if (ok(hipGetLastError()) && ok(hipMemcpyAsync(dst, dd, ncell * sizeof(double), hipMemcpyDeviceToHost, s)))
-            ok(hipStreamSynchronize(s));
+    if (ok(hipStreamCreateWithFlags(&s, hipStreamNonBlocking)) && (mem || ok(hipMalloc(&mem, plain)))) {
+        double *dc = (double*)mem, *dp = dc + 3 * ncell, *dd = dp + 3 * npanel;
+        if (ok(hipMemcpyAsync(dc, cells, 3 * ncell * sizeof(double), hipMemcpyHostToDevice, s)) &&
+            ok(hipMemcpyAsync(dp, panels, 3 * npanel * sizeof(double), hipMemcpyHostToDevice, s))) {
+            if (sorted)
+                launch_wb(s, dc, ncell, dp, npanel, dd);
+            else {
+                const long per = 256L * WD_CPT;
+                hipLaunchKernelGGL(k_wall_distance, dim3((unsigned)((ncell + per - 1) / per)), dim3(256), 0, s, dc,
+                                   ncell, dp, npanel, dd);
+            }
+            if (ok(hipGetLastError()) && ok(hipMemcpyAsync(dst, dd, ncell * sizeof(double), hipMemcpyDeviceToHost, s)))
+                ok(hipStreamSynchronize(s));
+        }
     }
-    if (dc) (void)hipFree(dc);
-    if (dp) (void)hipFree(dp);
-    if (dd) (void)hipFree(dd);
+    if (mem) (void)hipFree(mem);
     if (s) (void)hipStreamDestroy(s);
     if (rc) return rc;
     // sqrt of the clamped minimum (the reference clamps with tiny = 1e-20 between surfaces)
-    for (long c = 0; c < ncell; c++) dst[c] = std::sqrt(std::max(dst[c], 1.0e-20));
+    if (!sorted)
+        for (long c = 0; c < ncell; c++) dst[c] = std::sqrt(std::max(dst[c], 1.0e-20));
     return 0;
 }
 

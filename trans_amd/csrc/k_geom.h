@@ -293,3 +293,235 @@ __global__ void __launch_bounds__(256) k_geom_ghosts(GeomGrid g, GeomOut o)
         for (int x = 0; x < 3; x++) o.sd[2 + 3 * x + 9 * c] = o.sd[2 + 3 * x + 9 * s];
     }
 }
+
+// ---------------------------------------------------------------------------------------
+// The same minimum over fewer pairs, for many points: cells and panels are put in Morton order
+// (32^3 boxes of their bounding box, counting sort), panels in tiles of 64 with their bounding
+// boxes.  A wave holds 64 consecutive cells; it evaluates the tile that is nearest to
+// its cells' box, then every tile whose box is not farther than its largest minimum so far from its
+// cells' box, and then not farther from some cell than that cell's minimum.  A
+// skipped tile's pairs are all above the minima by more than their rounding (WB_SLACK), the pairs
+// evaluated are formed as above, and a minimum does not depend on the order, so the result is the
+// same bit for bit.  485 000 cells and 30 000 panels: 1.1 ms of kernels and 2.5 ms for the call, with
+// every pair 6 ms and 7.7 ms.  With two and four cells per lane 1.3 and 1.6 ms (larger boxes).
+constexpr int WB_BITS = 5, WB_BINS = 1 << (3 * WB_BITS);
+constexpr int WB_TILE = 64;
+constexpr double WB_SLACK = 1.0 + 1.0e-9;
+
+// Doubles as unsigned integers of the same order, for atomic minima and maxima.
+__device__ __forceinline__ unsigned long long wb_key(double x)
+{
+    const unsigned long long u = (unsigned long long)__double_as_longlong(x);
+    return u >> 63 ? ~u : u | (1ull << 63);
+}
+__device__ __forceinline__ double wb_unkey(unsigned long long u)
+{
+    return __longlong_as_double((long long)(u >> 63 ? u & ~(1ull << 63) : ~u));
+}
+
+// Two boxes (cells, panels) and their tables before the first point.
+__global__ void __launch_bounds__(256) k_wb_clear(unsigned long long* __restrict__ box, int* __restrict__ bins)
+{
+    const int q = blockIdx.x * 256 + threadIdx.x;
+    for (int k = q; k < 2 * WB_BINS; k += gridDim.x * 256) bins[k] = 0;
+    if (q < 12) box[q] = q % 6 < 3 ? ~0ull : 0ull;
+}
+
+// box: keys of the lower corner (3, initially all ones), then of the upper one (3, initially zero)
+__global__ void __launch_bounds__(256) k_wb_box(const double* __restrict__ pt, long n, unsigned long long* box)
+{
+    double lo[3], hi[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        lo[d] = INFINITY;
+        hi[d] = -INFINITY;
+    }
+    for (long q = (long)blockIdx.x * 256 + threadIdx.x; q < n; q += (long)gridDim.x * 256)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const double x = pt[d * n + q];
+            if (!isfinite(x)) continue;
+            lo[d] = fmin(lo[d], x);
+            hi[d] = fmax(hi[d], x);
+        }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            lo[d] = fmin(lo[d], __shfl_xor(lo[d], off, 64));
+            hi[d] = fmax(hi[d], __shfl_xor(hi[d], off, 64));
+        }
+    if (threadIdx.x % 64 == 0)
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+            if (lo[d] <= hi[d]) {
+                atomicMin(box + d, wb_key(lo[d]));
+                atomicMax(box + 3 + d, wb_key(hi[d]));
+            }
+}
+
+// Morton number of point q among the boxes of the bounding box.
+__device__ __forceinline__ int wb_bin(const double* __restrict__ pt, long n, long q, const unsigned long long* box)
+{
+    int m = 0;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const double lo = wb_unkey(box[d]), hi = wb_unkey(box[3 + d]);
+        const double s = (pt[d * n + q] - lo) / (hi - lo) * (1 << WB_BITS);
+        // (NaN, of a coordinate or of a flat box, takes the first)
+        const int k = (int)fmin(fmax(s, 0.0), (double)((1 << WB_BITS) - 1));
+#pragma unroll
+        for (int b = 0; b < WB_BITS; b++) m |= ((k >> b) & 1) << (3 * b + d);
+    }
+    return m;
+}
+
+__global__ void __launch_bounds__(256) k_wb_count(const double* __restrict__ pt, long n,
+                                                  const unsigned long long* __restrict__ box, int* __restrict__ bins)
+{
+    const long q = (long)blockIdx.x * 256 + threadIdx.x;
+    if (q < n) atomicAdd(bins + wb_bin(pt, n, q, box), 1);
+}
+
+// Counts to first positions; one workgroup per table.
+__global__ void __launch_bounds__(1024) k_wb_scan(int* __restrict__ tables)
+{
+    __shared__ int part[1024];
+    int* const t = tables + (long)blockIdx.x * WB_BINS;
+    constexpr int PER = WB_BINS / 1024;
+    int sum = 0;
+    for (int q = 0; q < PER; q++) sum += t[threadIdx.x * PER + q];
+    part[threadIdx.x] = sum;
+    __syncthreads();
+    for (int off = 1; off < 1024; off <<= 1) {
+        const int v = (int)threadIdx.x >= off ? part[threadIdx.x - off] : 0;
+        __syncthreads();
+        part[threadIdx.x] += v;
+        __syncthreads();
+    }
+    int at = part[threadIdx.x] - sum;
+    for (int q = 0; q < PER; q++) {
+        const int c = t[threadIdx.x * PER + q];
+        t[threadIdx.x * PER + q] = at;
+        at += c;
+    }
+}
+
+// Points to their sorted places: x, y, z, 0 per point, and where they came from (if asked for).
+__global__ void __launch_bounds__(256) k_wb_scatter(const double* __restrict__ pt, long n,
+                                                    const unsigned long long* __restrict__ box,
+                                                    int* __restrict__ bins, double4* __restrict__ out,
+                                                    int* __restrict__ from)
+{
+    const long q = (long)blockIdx.x * 256 + threadIdx.x;
+    if (q >= n) return;
+    const int at = atomicAdd(bins + wb_bin(pt, n, q, box), 1);
+    out[at] = make_double4(pt[q], pt[n + q], pt[2 * n + q], 0.0);
+    if (from) from[at] = (int)q;
+}
+
+// Bounding boxes of the panel tiles: 3 lower, 3 upper bounds, each ntile values; one wave per tile.
+__global__ void __launch_bounds__(64) k_wb_tiles(const double4* __restrict__ pan, int npan, int ntile,
+                                                 double* __restrict__ tb)
+{
+    const int q = min((int)(blockIdx.x * WB_TILE + threadIdx.x), npan - 1);
+    const double4 p = pan[q];
+    double lo[3] = {p.x, p.y, p.z}, hi[3] = {p.x, p.y, p.z};
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            lo[d] = fmin(lo[d], __shfl_xor(lo[d], off, 64));
+            hi[d] = fmax(hi[d], __shfl_xor(hi[d], off, 64));
+        }
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            tb[(long)d * ntile + blockIdx.x] = lo[d];
+            tb[(long)(3 + d) * ntile + blockIdx.x] = hi[d];
+        }
+}
+
+// One wave per workgroup: distances of 64 sorted cells.
+__global__ void __launch_bounds__(64) k_wb_distance(const double4* __restrict__ cell, const int* __restrict__ from,
+                                                    long ncell, const double4* __restrict__ pan, int npan,
+                                                    const double* __restrict__ tb, int ntile, double* __restrict__ dst)
+{
+    const int lane = threadIdx.x;
+    const long me = (long)blockIdx.x * 64 + lane;
+    const double4 c4 = cell[min(me, ncell - 1)];  // past the end: the last cell again
+    const double c[3] = {c4.x, c4.y, c4.z};
+    double best = 1.0e20;
+    double lo[3] = {c4.x, c4.y, c4.z}, hi[3] = {c4.x, c4.y, c4.z};
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            lo[d] = fmin(lo[d], __shfl_xor(lo[d], off, 64));
+            hi[d] = fmax(hi[d], __shfl_xor(hi[d], off, 64));
+        }
+    // squared distance between the box from a to b and that of tile t (a NaN counts as 0)
+    auto bound = [&](const double* a, const double* b, int t) {
+        double s = 0.0;
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const double x = fmax(fmax(tb[(long)d * ntile + t] - b[d], a[d] - tb[(long)(3 + d) * ntile + t]), 0.0);
+            s += x * x;
+        }
+        return s;
+    };
+    auto tile = [&](int t) {
+        const double4* const p = pan + (long)t * WB_TILE;
+        const int n = min(WB_TILE, npan - t * WB_TILE);
+#pragma unroll 4
+        for (int k = 0; k < n; k++) {
+            const double4 w = p[k];
+            const double dx = c[0] - w.x, dy = c[1] - w.y, dz = c[2] - w.z;
+            const double ddd = dx * dx + dy * dy + dz * dz;
+            best = ddd < best ? ddd : best;
+        }
+    };
+    auto worst = [&]() {
+        double m = best;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
+        return m * WB_SLACK;
+    };
+    // the nearest tile first
+    double near = INFINITY;
+    int first = 0;
+    for (int t = lane; t < ntile; t += 64) {
+        const double s = bound(lo, hi, t);
+        if (s < near) {
+            near = s;
+            first = t;
+        }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const double s = __shfl_xor(near, off, 64);
+        const int t = __shfl_xor(first, off, 64);
+        if (s < near || (s == near && t < first)) {
+            near = s;
+            first = t;
+        }
+    }
+    first = __builtin_amdgcn_readfirstlane(first);
+    tile(first);
+    double lim = worst();
+    for (int t0 = 0; t0 < ntile; t0 += 64) {
+        const double s = t0 + lane < ntile ? bound(lo, hi, t0 + lane) : INFINITY;
+        unsigned long long todo = __ballot(t0 + lane < ntile && t0 + lane != first && !(s > lim));
+        while (todo) {
+            const int b = __ffsll((long long)todo) - 1;
+            todo &= ~(1ull << b);
+            const int t = __builtin_amdgcn_readfirstlane(t0 + b);
+            if (!__any(!(bound(c, c, t) > best * WB_SLACK))) continue;
+            tile(t);
+            lim = worst();
+            todo &= __ballot(!(s > lim));  // what has come out of reach meanwhile
+        }
+    }
+    // the root of the clamped minimum, as the host forms it for the other form
+    if (me < ncell) dst[from[me]] = sqrt(fmax(best, 1.0e-20));
+}
