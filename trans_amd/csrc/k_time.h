@@ -70,7 +70,7 @@ __device__ __forceinline__ void lusgs_rhs_cell(const trans_params& p, const Fiel
     f1 = 1.0 + (f.Rds[c] + f.Rds[tot + c] + f.Rds[2 * tot + c]) * cvs;
 }
 
-// The 17 values the line-march and tile sweeps read from the hyperplane-major buffer, written
+// The 17 values the sweeps on the hyperplane-major buffer read from it, written
 // by the right-hand side, with their components: D(1:5), stept, cvs, stept/F1, cvs/F1, 1/rho,
 // u, v, w, p, Rds(1:3).
 constexpr int RHS_NW = 17;
@@ -429,8 +429,8 @@ __global__ void __launch_bounds__(1024) k_lusgs_sweep(trans_params p, Fields f, 
 }
 
 // ---------------------------------------------------------------------------------------
-// Line-march wavefront of the same sweeps.  The block is cut into lines along a march axis
-// MARCH (j when the (i,k) cross-section fits one workgroup).  At step t the thread of line
+// Line-march wavefront of the same sweeps (selected by tuning only).  The block is cut into lines
+// along a march axis MARCH, i or k (0, 2), whose cross-section fits one workgroup.  At step t the thread of line
 // (a,b) updates the cell of its line on hyperplane s = (i-1)+(j-1)+(k-1).  After updating its
 // increment a cell evaluates the three terms its downstream neighbours need,
 // 0.5*(A_d dQ +/- Rds_d dQ) (exactly the expressions of Time/TIME_LUSGS.F90:190-256 the
@@ -557,7 +557,8 @@ __device__ __forceinline__ void line_sweep(const Fields& f, R* __restrict__ Dq, 
     static_assert(NEQ == 5 || NEQ == 2, "mean flow or k-omega");
     constexpr bool MF = NEQ == 5;
     const int NI1 = b.ni - 1, NJ1 = b.nj - 1, NK1 = b.nk - 1;
-    const int Nm = MARCH == 0 ? NI1 : (MARCH == 1 ? NJ1 : NK1);
+    static_assert(MARCH == 0 || MARCH == 2, "along i or k");
+    const int Nm = MARCH == 0 ? NI1 : NK1;
     const int Na = MARCH == 0 ? NJ1 : NI1;
     const int Nb = MARCH == 2 ? NJ1 : NK1;
     const int nlines = Na * Nb;
@@ -609,8 +610,6 @@ __device__ __forceinline__ void line_sweep(const Fields& f, R* __restrict__ Dq, 
             R sum;
             if constexpr (MARCH == 0)
                 sum = sm + sa + sb;
-            else if constexpr (MARCH == 1)
-                sum = sa + sm + sb;
             else
                 sum = sa + sb + sm;
             if constexpr (MF) {

@@ -1499,7 +1499,7 @@ static int rk_update_async(trans_ctx* c, int stage)
     return launch_check(c, "rk_update");
 }
 
-// The error flag of the tile wavefront's bounded waits (read once the stream is idle).
+// The error flag of the wave sweeps' bounded waits (read once the stream is idle).
 static int check_sweep_flag(trans_ctx* c)
 {
     if (!c->d_err) return 0;
