@@ -39,8 +39,8 @@ def alg_bytes(name, neq, fp32, dual_shift=True):
     r = 4 if fp32 else 8
     turb = neq == 7
     table = {
-        # V(1:4), PP, T, Rmiu, Vol, SD (9 face values per cell) in; Rds(3), Dtm out
-        "k_spectral_radius": ("cell", d * (4 + 1 + 1 + 1 + 1 + 9 + 3 + 1) + (4 * 3 if fp32 else 0)),
+        # V(1:4[,6:7]), PP, T, Rmiu, Vol, SD (9 face values per cell) in; Rds(3), Dtm, Q(3[,5]) out
+        "k_spectral_radius": ("cell", d * (4 + 1 + 1 + 1 + 1 + 9 + 3 + 1 + (7 if turb else 3)) + (4 * 3 if fp32 else 0)),
         # V(1:4[,6:7]) in; Q(3[,5]) out
         "k_prim_cells": ("cell", d * ((6 if turb else 4) + (5 if turb else 3))),
         # Q(3[,5]), T, Alagm(3), SD(9), Vol in; DQ(12[,18]), shock out
