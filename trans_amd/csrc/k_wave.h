@@ -29,11 +29,11 @@
 // (NJ1 + tile diagonals x the skew) x row time; with many, the memory system (144 B/cell FP32 per
 // sweep).  Forward and backward sweep together, before (one workgroup per block marching lines
 // with a barrier per step, or tiles of 256 lines with progress counters) and now:
-//     65k-cell bump channel, FP64           707 us   236 us
-//     131k-cell plate, FP64 k-omega         406 us   237 us
-//     0.13M-cell sector, FP64 k-omega       263 us   103 us
-//     0.49M-cell sector, FP32 k-omega       395 us   179 us
-//     8.1M-cell sector, FP32 k-omega       2129 us  1169 us
+//     65k-cell bump channel, FP64           707 us   218 us
+//     131k-cell plate, FP64 k-omega         406 us   225 us
+//     0.13M-cell sector, FP64 k-omega       263 us    97 us
+//     0.49M-cell sector, FP32 k-omega       395 us   164 us
+//     8.1M-cell sector, FP32 k-omega       2129 us  1060 us
 // Tiles of 16 x 4 lines: the i terms then stay within a DPP row of 16 lanes.
 #pragma once
 #include "k_time.h"

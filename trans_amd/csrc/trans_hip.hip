@@ -1317,7 +1317,8 @@ static void launch_wave_sweeps(trans_ctx* c)
 // From four tiles per CU on (1024) the FP32 sweeps keep four rows of a wave in flight at two waves
 // per SIMD: 1169 us for both sweeps of the 8.1M-cell sector (1760 tiles, k-omega) instead of
 // 1307 us with two rows at four waves.  Below, a row's latency counts more than its loads: 179 us
-// against 201 us at 0.49M cells (392 tiles), 132 us against 134 us on a 25 k-cell plate (25 tiles).
+// against 201 us at 0.49M cells (392 tiles), 132 us against 134 us on a 25 k-cell plate (25 tiles)
+// (all while a poll waited for one row only; 1060, 164 and 115 us since).
 // The FP64 k-omega sweeps alone have the registers for a third row (334 us against 414 us for the
 // three stages of a 0.30M-cell cascade); with the mean flow two rows are as good (103 us against
 // 113 us at 0.13M cells).
