@@ -529,16 +529,34 @@ static void launch_face_means(trans_ctx* c, int seg0, int nseg)
 
 // Selects the LU-SGS sweep: m = 1 or 3 the wave sweeps along j (tile packets), m = 0 or 2 the line
 // march along that axis (hyperplane-major buffer W or Wf), m = -2 one launch per hyperplane (the
-// same buffer, march axis j), m = -1 the hyperplane kernel on the natural layout.
+// same buffer, march axis j), m = -1 the hyperplane kernel on the natural layout.  What is refused
+// leaves the context as it was.
 static int set_sweep(trans_ctx* c, int m, bool upload)
 {
     int mx = 0;
-    // the low-Mach preconditioning transforms live in the natural-layout hyperplane sweep
+    // the preconditioning transform is implemented in the hyperplane sweep only
     if (c->p.if_precondition && m != -1)
         return fail(c, TRANS_EUNSUPPORTED, "with IF_PRECONDITION = 1 only the hyperplane sweep (-1) runs");
     if (m < -2 || m > 3) return fail(c, TRANS_EINVAL, "sweep must be -2, -1, 0, 1, 2 or 3");
     if (m >= 0 && m <= 2 && !march_fits(c, m, &mx))
         return fail(c, TRANS_EINVAL, "the line sweep does not fit this axis");
+    const int axis = m == 0 || m == 2 ? m : 1;
+    // hyperplane-major sweep buffer: nplanes x nlines slots per block, then per
+    // component a sink of 1024 slots for each of the 2 workgroups of every block
+    long wt = 0, rows = 0;
+    bool rows_ok = true;  // a wave addresses its tile's rows with 31-bit byte offsets
+    for (const HostBlock& h : c->hb) {
+        const int n[3] = {h.ni - 1, h.nj - 1, h.nk - 1};
+        wt += (long)(n[0] + n[1] + n[2] - 2) * n[(axis + 1) % 3] * n[(axis + 2) % 3];
+        rows += wave_block_rows(h);
+        rows_ok = rows_ok && (long)wave_rows(h.nj) * WaveRow<double>::BYTES < (1L << 31);
+    }
+    const long sink = wt;
+    wt += (long)c->hb.size() * 2 * 1024;
+    const bool wave = (m == 1 || m == 3) && rows_ok;
+    // the sweeps on the hyperplane-major buffer address a component with 32-bit byte offsets
+    if (m != -1 && !wave && wt * (long)sizeof(double) >= (1L << 32))
+        return fail(c, TRANS_EUNSUPPORTED, "too many cells for the hyperplane-major sweep buffer");
     free_tiles(c);
     if (c->wbuf) {
         if (!c->dry) (void)hipFree(c->wbuf);
@@ -556,25 +574,11 @@ static int set_sweep(trans_ctx* c, int m, bool upload)
     c->sweep_mode = -1;
     const size_t esz = c->p.implicit_fp32 ? sizeof(float) : sizeof(double);
     if (m != -1) {
-        c->march = m == 0 || m == 2 ? m : 1;
-        // hyperplane-major sweep buffer: nplanes x nlines slots per block, then per
-        // component a sink of 1024 slots for each of the 2 workgroups of every block
-        long wt = 0, rows = 0;
-        bool rows_ok = true;  // a wave addresses its tile's rows with 31-bit byte offsets
-        for (const HostBlock& h : c->hb) {
-            const int n[3] = {h.ni - 1, h.nj - 1, h.nk - 1};
-            wt += (long)(n[0] + n[1] + n[2] - 2) * n[(c->march + 1) % 3] * n[(c->march + 2) % 3];
-            rows += wave_block_rows(h);
-            rows_ok = rows_ok && (long)wave_rows(h.nj) * WaveRow<double>::BYTES < (1L << 31);
-        }
-        f.wsink = wt;
-        wt += (long)c->hb.size() * 2 * 1024;
-        // the sweep addresses a component with 32-bit byte offsets
-        if (wt * (long)sizeof(double) >= (1L << 32))
-            return fail(c, TRANS_EUNSUPPORTED, "too many cells for the line-march sweep buffer");
-        c->wave = (m == 1 || m == 3) && rows_ok;
+        c->march = axis;
+        f.wsink = sink;
+        c->wave = wave;
         c->wave_alt = march_fits(c, 0, nullptr) || march_fits(c, 1, nullptr) || march_fits(c, 2, nullptr);
-        c->plane_launch = m == -2 || ((m == 1 || m == 3) && !rows_ok);
+        c->plane_launch = m == -2 || ((m == 1 || m == 3) && !wave);
         if (m == 0 || m == 2) {
             c->max_lines = mx;
             c->line_threads = (mx + 63) / 64 * 64;

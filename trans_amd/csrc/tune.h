@@ -64,7 +64,12 @@ int trans_hip_autotune(trans_ctx* c, int iters, trans_tune_entry* out, int max_o
         if (rc) break;
         if (sw >= 0 && sw <= 2 && !march_fits(c, sw, nullptr)) continue;
         if (c->p.if_precondition && sw != -1) continue;  // the transform lives in the hyperplane sweep
-        if ((rc = set_sweep(c, sw, true))) break;
+        rc = set_sweep(c, sw, true);
+        if (rc == TRANS_EUNSUPPORTED) {  // too many cells for this candidate's buffer
+            rc = 0;
+            continue;
+        }
+        if (rc) break;
         for (int st = 0; st < 2 && !rc; st++) {
             if (st == 0 && !c->aux_own[0]) continue;  // single-stream context
             apply_streams(c, st == 1);
