@@ -509,9 +509,10 @@ static int build_tiles(trans_ctx* c)
     c->tile_bytes = tab.size() * sizeof(WaveTile) + ebytes + 2 * sizeof(int);
     c->bytes += c->tile_bytes;
     if (c->dry) return 0;
-    HIPCHK(c, hipMalloc(&c->d_tiles, tab.size() * sizeof(WaveTile)));
-    HIPCHK(c, hipMalloc(&c->wave_edge, ebytes));
-    HIPCHK(c, hipMalloc(&c->d_tctr, 2 * sizeof(int)));
+    hipError_t e = hipMalloc(&c->d_tiles, tab.size() * sizeof(WaveTile));
+    if (e == hipSuccess) e = hipMalloc(&c->wave_edge, ebytes);
+    if (e == hipSuccess) e = hipMalloc(&c->d_tctr, 2 * sizeof(int));
+    if (e != hipSuccess) return fail(c, TRANS_ENOMEM, std::string("sweep buffer: ") + hipGetErrorString(e));
     return h2d(c, c->d_tiles, tab.data(), tab.size() * sizeof(WaveTile));
 }
 
@@ -527,10 +528,31 @@ static void launch_face_means(trans_ctx* c, int seg0, int nseg)
         hipLaunchKernelGGL(k_face_means, dim3(nseg), dim3(WG), 0, c->stream, c->f, c->d_blk, seg);
 }
 
+// Gives the sweep's buffers back: what stays is the hyperplane kernel on the natural layout (-1),
+// which needs none.
+static void drop_sweep(trans_ctx* c)
+{
+    drop_graph(c);
+    free_tiles(c);
+    if (c->wbuf && !c->dry) (void)hipFree(c->wbuf);
+    c->wbuf = nullptr;
+    if (!c->dry) (void)hipGetLastError();  // of the allocation that failed, if one did
+    c->bytes -= c->wbytes;
+    c->wbytes = 0;
+    c->f.W = nullptr;
+    c->f.Wf = nullptr;
+    c->f.P = nullptr;
+    c->line_threads = 0;
+    c->wave = false;
+    c->plane_launch = false;
+    c->plain = false;
+    c->sweep_mode = -1;
+}
+
 // Selects the LU-SGS sweep: m = 1 or 3 the wave sweeps along j (tile packets), m = 0 or 2 the line
 // march along that axis (hyperplane-major buffer W or Wf), m = -2 one launch per hyperplane (the
 // same buffer, march axis j), m = -1 the hyperplane kernel on the natural layout.  What is refused
-// leaves the context as it was.
+// leaves the context as it was; where a buffer cannot be allocated, it is left with -1.
 static int set_sweep(trans_ctx* c, int m, bool upload)
 {
     int mx = 0;
@@ -557,25 +579,30 @@ static int set_sweep(trans_ctx* c, int m, bool upload)
     // the sweeps on the hyperplane-major buffer address a component with 32-bit byte offsets
     if (m != -1 && !wave && wt * (long)sizeof(double) >= (1L << 32))
         return fail(c, TRANS_EUNSUPPORTED, "too many cells for the hyperplane-major sweep buffer");
-    free_tiles(c);
-    if (c->wbuf) {
-        if (!c->dry) (void)hipFree(c->wbuf);
-        c->wbuf = nullptr;
-    }
-    c->bytes -= c->wbytes;
-    c->wbytes = 0;
+    drop_sweep(c);
     Fields& f = c->f;
-    f.W = nullptr;
-    f.Wf = nullptr;
-    f.P = nullptr;
-    c->line_threads = 0;
-    c->wave = false;
-    c->plane_launch = false;
-    c->sweep_mode = -1;
-    const size_t esz = c->p.implicit_fp32 ? sizeof(float) : sizeof(double);
     if (m != -1) {
-        c->march = axis;
+        const size_t esz = c->p.implicit_fp32 ? sizeof(float) : sizeof(double);
+        const size_t bytes = wave ? (size_t)rows * WaveRow<double>::ELEMS * esz : (size_t)W_NCOMP * wt * esz;
+        if (!c->dry) {
+            hipError_t e = hipMalloc(&c->wbuf, bytes);
+            if (e == hipSuccess && !wave) e = hipMemsetAsync(c->wbuf, 0, bytes, c->stream);
+            if (e != hipSuccess) {
+                drop_sweep(c);
+                return fail(c, TRANS_ENOMEM, std::string("sweep buffer: ") + hipGetErrorString(e));
+            }
+        }
+        c->wbytes = bytes;
+        c->bytes += bytes;
+        c->march = f.march = axis;
+        f.wtot = wt;
         f.wsink = sink;
+        if (wave)
+            f.P = c->wbuf;
+        else if (c->p.implicit_fp32)
+            f.Wf = (float*)c->wbuf;
+        else
+            f.W = (double*)c->wbuf;
         c->wave = wave;
         c->wave_alt = march_fits(c, 0, nullptr) || march_fits(c, 1, nullptr) || march_fits(c, 2, nullptr);
         c->plane_launch = m == -2 || ((m == 1 || m == 3) && !wave);
@@ -583,36 +610,21 @@ static int set_sweep(trans_ctx* c, int m, bool upload)
             c->max_lines = mx;
             c->line_threads = (mx + 63) / 64 * 64;
         }
-        f.wtot = wt;
-        f.march = c->march;
-        const size_t bytes = c->wave ? (size_t)rows * WaveRow<double>::ELEMS * esz : (size_t)W_NCOMP * wt * esz;
-        if (!c->dry) {
-            hipError_t e = hipMalloc(&c->wbuf, bytes);
-            if (e != hipSuccess) return fail(c, TRANS_ENOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-            if (!c->wave) HIPCHK(c, hipMemsetAsync(c->wbuf, 0, bytes, c->stream));
-        }
-        c->wbytes = bytes;
-        c->bytes += bytes;
-        if (c->wave)
-            f.P = c->wbuf;
-        else if (c->p.implicit_fp32)
-            f.Wf = (float*)c->wbuf;
-        else
-            f.W = (double*)c->wbuf;
-    }
-    if (c->wave) {
-        int rc = build_tiles(c);
-        if (rc) return rc;
     }
     c->sweep_mode = m;
-    drop_graph(c);
-    if (!upload) return 0;
-    int rc = upload_blk_table(c);
-    if (rc || m == -1 || c->dry) return rc;
+    int rc = wave ? build_tiles(c) : 0;
+    if (!rc && upload) rc = upload_blk_table(c);
+    if (rc) {
+        drop_sweep(c);
+        return rc;
+    }
+    if (!upload || m == -1 || c->dry) return 0;
     // the geometry part of the new buffer (face means, written once per geometry upload)
     launch_face_means(c, 0, c->seg_cell.n);
-    HIPCHK(c, hipGetLastError());
-    return 0;
+    const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) return 0;
+    drop_sweep(c);
+    return fail(c, TRANS_EHIP, std::string("face means: ") + hipGetErrorString(e));
 }
 
 // dry: sizing run only.  single_stream: the helper streams are the context's own stream, so

@@ -106,7 +106,7 @@ int trans_hip_autotune(trans_ctx* c, int iters, trans_tune_entry* out, int max_o
         rc2 = set_sweep(c, sweep0, true);
         apply_streams(c, single0);
         c->graphs = graphs0;
-        c->plain = plain0;
+        if (!rc2) c->plain = plain0;
     }
     if (!rc2) rc2 = copy_state(true);
     if (!rc2) {
