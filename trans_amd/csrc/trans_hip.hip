@@ -242,6 +242,24 @@ static void join_aux(trans_ctx* c, int n)
     }
 }
 
+// A fork of helper stream 0 that is joined on every way out.
+struct AuxScope {
+    trans_ctx* c;
+    bool open = false;
+    explicit AuxScope(trans_ctx* ctx) : c(ctx) {}
+    ~AuxScope() { join(); }
+    void fork()
+    {
+        fork_aux(c, 1);
+        open = true;
+    }
+    void join()
+    {
+        if (open) join_aux(c, 1);
+        open = false;
+    }
+};
+
 static void drop_graph(trans_ctx* c)
 {
     if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
@@ -1203,8 +1221,9 @@ static int space_async(trans_ctx* c, bool prim)
     // (131k-cell plate) with MDCD, 806 -> 801 us (0.49M-cell sector) with MUSCL.
     const bool side = visc && !fused;
     const bool early = c->p.kind_spatial <= 2 && c->p.kind_roe != 2;
+    AuxScope aux(c);
     auto conv_aside = [&]() {
-        fork_aux(c, 1);
+        aux.fork();
         launch_conv(c, c->aux[0], if_turb, 0, nblk);
     };
     if (side && early) conv_aside();
@@ -1227,7 +1246,7 @@ static int space_async(trans_ctx* c, bool prim)
         KLAUNCH(c, "k_visc_faces", k_visc_faces, dim3(3 * c->brick_face.n(0, nblk)), dim3(WG), c->p, if_turb, c->f,
                 c->d_blk, c->brick_face.d);
     if (side)
-        join_aux(c, 1);
+        aux.join();
     else
         launch_conv(c, c->stream, if_turb, 0, nblk);
     KLAUNCH(c, "k_accumulate_visc", k_accumulate_visc, dim3(c->seg_cell.n), dim3(WG), c->p, c->p.if_euler,
@@ -1246,9 +1265,9 @@ int trans_hip_residual(trans_ctx* c)
     int rc;
     // The outlet march reads interior cells only and writes only its own ghosts, so it runs
     // beside the spectral radius and the other patches' BC (which copies its Rds ghosts).
-    const bool outl = c->n_outl > 0;
-    if (outl) {
-        fork_aux(c, 1);
+    AuxScope aux(c);
+    if (c->n_outl) {
+        aux.fork();
         KLAUNCH_ON(c, c->aux[0], "k_bc_outlet", k_bc_outlet, dim3(c->n_outl), dim3(256), c->p, if_turb_now(c), c->f,
                    c->d_blk, c->d_patch, c->d_outl);
     }
@@ -1258,7 +1277,7 @@ int trans_hip_residual(trans_ctx* c)
     if (c->n_bcseg)
         KLAUNCH(c, "k_bc", k_bc, dim3(c->n_bcseg), dim3(128), c->p, if_turb_now(c), -1, c->f, c->d_blk, c->d_patch,
                 c->d_bcseg);
-    if (outl) join_aux(c, 1);
+    aux.join();
     if ((rc = launch_check(c, "k_bc"))) return rc;
     return space_async(c, false);
 }
