@@ -321,8 +321,10 @@ int trans_tecplot_write_ascii(const char* path, const char* title, const char* z
  * buffer is reallocated for the chosen axis, so the context's device bytes may then differ
  * from trans_hip_footprint's.  get_tuning reports the configuration in use. */
 typedef struct trans_tune_entry {
-    int sweep;     /* 0, 2 line march along i, k; 1, 3 tile wavefront along j; -2 one launch per hyperplane;
-                      -1 one workgroup per block; -3 plain drop-in schedule (set_tuning only) */
+    int sweep;     /* 0, 2 line march along i, k; 1, 3 tile wavefront along j (reported as -2,
+                      which then runs, beyond about 144 000 points along j); -2 one launch per
+                      hyperplane; -1 one workgroup per block; -3 plain drop-in schedule
+                      (set_tuning only) */
     int streams;
     int graph;
     double ms_per_iter;

@@ -6,6 +6,8 @@ import pytest
 
 from trans_amd import capi, cases, serving, solver
 
+from stub_lib import events, stub  # noqa: F401
+
 
 def _footprint(size, fp32):
     blocks, org, glob = cases.flat_plate(nblk=1, ni_total=33, nj=17, nk=4, lo=9, hi=33)
@@ -30,3 +32,29 @@ def test_long_blocks_are_taken(size, fp32):
     assert rc == 0
     cells = n[0] * n[1] * n[2]
     assert nbytes < 4000 * cells
+
+
+def test_tuning_reports_the_sweep_that_runs(stub):
+    """A wave addresses its tile's rows with 31-bit offsets: beyond about 144 000 points along j
+    the sweeps run one launch per hyperplane, and the tuning says so."""
+    blocks, org, glob = cases.flat_plate(nblk=1, ni_total=33, nj=17, nk=4, lo=9, hi=33)
+    prm = solver.prepare_case(blocks, org, glob)
+    descs, keep = serving._descs(blocks)
+    descs[0].npatch = 0
+    lib = capi.load_library()
+    for nj, want in ((17, 1), (140_000, 1), (150_000, -2)):
+        descs[0].ni, descs[0].nj, descs[0].nk = 4, nj, 4
+        ctx, t = C.c_void_p(), capi.TransTuneEntry()
+        assert lib.trans_hip_create(C.byref(prm), 1, descs, C.byref(ctx)) == 0
+        for sweep in (None, 3, 1):
+            if sweep:
+                t = capi.TransTuneEntry(sweep, 1, 0, 0.0, 16, 16, 8)
+                assert lib.trans_hip_set_tuning(ctx, C.byref(t)) == 0
+            assert lib.trans_hip_get_tuning(ctx, C.byref(t)) == 0
+            assert t.sweep == (want if want < 0 else sweep or want), (nj, sweep)
+        lib.stub_reset()
+        assert lib.trans_hip_lusgs_update(ctx, None) == 0
+        names = [nm for what, nm, _ in events(lib) if what == "launch"]
+        assert any("k_lusgs_wave" in nm for nm in names) == (want == 1)
+        assert any("k_lusgs_wplane" in nm for nm in names) == (want == -2)
+        lib.trans_hip_destroy(ctx)

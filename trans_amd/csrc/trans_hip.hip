@@ -123,7 +123,7 @@ struct trans_ctx {
     // item counters, and the error flag of the bounded waits
     bool wave = false;
     bool wave_alt = false;  // round as the line march, which these blocks fit
-    int sweep_mode = -1;  // the mode asked for (cur_sweep)
+    int sweep_mode = -1;  // the mode in use (cur_sweep)
     int tile_a = 16, tile_b = 16, tile_chunk = 8;  // of the last set_tuning
     WaveTile* d_tiles = nullptr;
     int ntiles = 0;
@@ -567,7 +567,7 @@ static void drop_sweep(trans_ctx* c)
 
 // Selects the LU-SGS sweep: m = 1 or 3 the wave sweeps along j (tile packets), m = 0 or 2 the line
 // march along that axis (hyperplane-major buffer W or Wf), m = -2 one launch per hyperplane (the
-// same buffer, march axis j), m = -1 the hyperplane kernel on the natural layout.  What is refused
+// same buffer, march axis j; also for 1 and 3 where a tile's rows are too long for them), m = -1 the hyperplane kernel on the natural layout.  What is refused
 // leaves the context as it was; where a buffer cannot be allocated, it is left with -1.
 static int set_sweep(trans_ctx* c, int m, bool upload)
 {
@@ -621,7 +621,8 @@ static int set_sweep(trans_ctx* c, int m, bool upload)
             f.W = (double*)c->wbuf;
         c->wave = wave;
         c->wave_alt = march_fits(c, 0, nullptr) || march_fits(c, 1, nullptr) || march_fits(c, 2, nullptr);
-        c->plane_launch = m == -2 || ((m == 1 || m == 3) && !wave);
+        if ((m == 1 || m == 3) && !wave) m = -2;
+        c->plane_launch = m == -2;
         if (m == 0 || m == 2) {
             c->max_lines = mx;
             c->line_threads = (mx + 63) / 64 * 64;

@@ -71,6 +71,7 @@ int trans_hip_autotune(trans_ctx* c, int iters, trans_tune_entry* out, int max_o
             continue;
         }
         if (rc) break;
+        if (cur_sweep(c) != sw) continue;  // it runs one launch per hyperplane, a candidate of its own
         for (int st = 0; st < 2 && !rc; st++) {
             if (st == 0 && !c->aux_own) continue;  // single-stream context
             apply_streams(c, st == 1);
