@@ -930,6 +930,11 @@ static int copy_views(trans_ctx* c, int blk, const ViewJob* jobs, int njobs, boo
         double* host;
         long vrow, vplane;  // host strides of a row and of a plane (values)
         bool dense;         // the box is one range of the view
+        const double* last() const
+        {
+            const int n2 = b.cells / (b.n0 * b.n1);
+            return host + (n2 - 1) * vplane + (b.n1 - 1) * vrow + (long)b.n0 * b.ncomp - 1;
+        }
     };
     std::vector<Slab> slabs;
     const long cap = 7 * c->tot;  // of each flux array
@@ -1015,6 +1020,13 @@ static int copy_views(trans_ctx* c, int blk, const ViewJob* jobs, int njobs, boo
             s.vrow = vrow;
             s.vplane = vplane;
             s.dense = (long)nc * n0 == vrow && ((long)n1 * vrow == vplane || n2 == 1);
+            // (host threads fill the boxes in any order: a later one that overlaps waits its turn)
+            bool again = false;
+            for (const Slab& q : slabs) again = again || (!upload && s.host <= q.last() && q.host <= s.last());
+            if (again) {
+                if ((rc = flush())) return rc;
+                continue;
+            }
             if (!upload)
                 hipLaunchKernelGGL(k_view<false>, dim3((s.b.cells + WG - 1) / WG), dim3(WG), 0, c->stream, s.b);
             slabs.push_back(s);
