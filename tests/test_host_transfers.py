@@ -59,3 +59,39 @@ def test_views_of_one_array_are_filled_in_order(stub):
     read(v=at(0), wt0=at(half))
     assert 0 < long[:half].min() and long[:half].max() <= first and long[half:].min() > first
     sv.close()
+
+
+@pytest.mark.parametrize("call", ["get_state", "set_state", "get_field"])
+def test_no_host_memory_is_an_error_code(stub, call):
+    """Wherever host memory runs out in a transfer (lists, gather buffers, threads), the call
+    returns TRANS_ENOMEM, every thread has ended and the pinned buffers are back."""
+    sv = _solver(45)
+    b = sv.blocks[0]
+    # views of wider arrays, so that rows are gathered and scattered on the host
+    wide = tuple(n + 2 for n in b.shape())
+    host = {nm: np.zeros((nc,) + wide if nc > 1 else wide, order="F") for nm, nc in (("v", 7), ("pp", 1), ("wt0", 7))}
+    s = capi.TransStateView()
+    for nm, a in host.items():
+        setattr(s, nm, capi.fview(a, lo=(-3, -3, -3)))
+
+    def go():
+        if call == "get_field":
+            return sv.lib.trans_hip_get_field(sv.ctx, 0, capi.FIELD_D, C.byref(s.v))
+        return getattr(sv.lib, "trans_hip_" + call)(sv.ctx, 0, C.byref(s))
+    assert go() == 0
+    pinned = stub.stub_mapped()
+    n = 0
+    while True:
+        stub.stub_fail_new(n)
+        rc = go()
+        left = stub.stub_new_left()
+        stub.stub_fail_new(-1)
+        assert rc in (0, capi.TRANS_ENOMEM), (n, rc)
+        if left > 0:  # more than the call needs
+            assert rc == 0
+            break
+        n += 1
+    assert n > 5  # (the first attempts had failed)
+    assert go() == 0
+    assert stub.stub_mapped() == pinned
+    sv.close()

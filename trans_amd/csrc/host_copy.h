@@ -9,8 +9,9 @@
 #pragma once
 #include <algorithm>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -76,8 +77,11 @@ struct PinPool {
         {
             std::lock_guard<std::mutex> g(m);
             if (users > 0 && (int)idle.size() < HC_POOL) {
-                idle.push_back(b);
-                return;
+                try {
+                    idle.push_back(b);
+                    return;
+                } catch (const std::bad_alloc&) {  // not kept
+                }
             }
         }
         drop(b);
@@ -168,7 +172,8 @@ static hipError_t host_copy_pieces(const std::vector<HostCopy>& list, const std:
 }
 
 // The copies, after the stream's work so far.  Downloads are complete on return, uploads are queued
-// on the stream and no longer read the host's memory.
+// on the stream and no longer read the host's memory.  (May throw std::bad_alloc, with no
+// buffer kept and no thread running.)
 static hipError_t host_copies(const std::vector<HostCopy>& list, bool upload, hipStream_t stream)
 {
     size_t total = 0;
@@ -181,10 +186,20 @@ static hipError_t host_copies(const std::vector<HostCopy>& list, bool upload, hi
     if (total >= HC_MIN) {
         pieces = host_pieces(list);
         const int want = 2 * (int)std::min<size_t>(HC_THREADS, pieces.size());
+        bufs.reserve((size_t)want);
         PinBuf b;
         while ((int)bufs.size() < want && g_pins.take(dev, b)) bufs.push_back(b);
     }
     const int nt = (int)bufs.size() / 2;
+    std::vector<std::thread> th;
+    std::vector<hipError_t> er;
+    try {
+        th.reserve((size_t)nt);
+        er.resize((size_t)nt, hipSuccess);
+    } catch (const std::bad_alloc&) {
+        for (const PinBuf& b : bufs) g_pins.give(b);
+        throw;
+    }
     if (nt == 0) {
         for (const HostCopy& c : list) {
             e = upload ? hipMemcpyAsync(c.dev, c.host, c.bytes, hipMemcpyHostToDevice, stream)
@@ -194,15 +209,13 @@ static hipError_t host_copies(const std::vector<HostCopy>& list, bool upload, hi
         const hipError_t r = hipStreamSynchronize(stream);
         if (e == hipSuccess) e = r;
     } else {
-        std::vector<std::thread> th;
-        std::vector<hipError_t> er((size_t)nt, hipSuccess);
         int started = 1;
         try {
             for (; started < nt; started++)
                 th.emplace_back([&, t = started] {
                     er[(size_t)t] = host_copy_pieces(list, pieces, t, nt, upload, dev, stream, &bufs[2 * (size_t)t]);
                 });
-        } catch (const std::system_error&) {  // no more threads: the caller does their pieces
+        } catch (const std::exception&) {  // no more threads, or no memory for one: the caller does their pieces
         }
         er[0] = host_copy_pieces(list, pieces, 0, nt, upload, dev, stream, &bufs[0]);
         for (int t = started; t < nt; t++)

@@ -7,10 +7,9 @@
 
 #include <algorithm>
 #include <cstdio>
-#include <map>
-#include <tuple>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -222,6 +221,16 @@ static int fail(trans_ctx* c, int code, const std::string& msg)
 {
     if (c) c->err = msg;
     return code;
+}
+
+static int no_host_memory(trans_ctx* c)
+{
+    try {
+        c->err = "out of host memory";
+    } catch (const std::bad_alloc&) {
+        c->err.clear();
+    }
+    return TRANS_ENOMEM;
 }
 
 // The helper stream waits for the work queued so far on the context's stream.
@@ -921,7 +930,7 @@ struct ViewJob {
 // (1.6 MB) 361, 196 and now 145 us; setting the state of a 0.2M-cell block (78 MB) 15.7, 2.7 and
 // now 2.2 ms.
 static int copy_views(trans_ctx* c, int blk, const ViewJob* jobs, int njobs, bool upload)
-{
+try {
     const HostBlock& h = c->hb[blk];
     const int dims[3] = {h.ni, h.nj, h.nk};
     // slabs that are on their way: the box, the host address of its first cell and the strides
@@ -1035,6 +1044,8 @@ static int copy_views(trans_ctx* c, int blk, const ViewJob* jobs, int njobs, boo
         }
     }
     return flush();
+} catch (const std::bad_alloc&) {  // (no exception may reach the caller, who need not be C++)
+    return no_host_memory(c);
 }
 
 static int copy_view(trans_ctx* c, int blk, const trans_fview& v, double* dbase, int ncomp, bool upload)
