@@ -342,7 +342,8 @@ int trans_hip_get_tuning(const trans_ctx* ctx, trans_tune_entry* out);
  * batched schedule.  Decks without preconditioning only (TRANS_EUNSUPPORTED otherwise).  A
  * baseline for the batched schedule; autotune leaves it for the batched candidates.
  * A tile-wavefront sweep whose wait for another tile exceeds its spin limit (a schedule that cannot
- * advance) ends and makes the next synchronising call return TRANS_ETIMEOUT.
+ * advance) ends, and the next call that hands results out (norms, a state, a field, statistics,
+ * integrals, a file) or synchronises returns TRANS_ETIMEOUT, once; a served solve fails with it.
  * A refused configuration leaves the context as it was; where a sweep's buffers cannot be
  * allocated (TRANS_ENOMEM) the context goes on with sweep -1, which needs none. */
 int trans_hip_set_tuning(trans_ctx* ctx, const trans_tune_entry* t);

@@ -56,7 +56,7 @@ extern "C" {
 int trans_hip_write_restart(trans_ctx* c, int blk, int ki, const char* path)
 {
     if (!c || !path || blk < 0 || blk >= (int)c->hb.size()) return TRANS_EINVAL;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (int rc = sync_results(c)) return rc;
     FILE* fp = std::fopen(path, "wb");
     if (!fp) return fail(c, TRANS_EINVAL, std::string("cannot open ") + path);
     const int32_t k32 = ki;
@@ -150,7 +150,7 @@ int trans_hip_get_stats(trans_ctx* c, int blk, const trans_fview* out)
 {
     if (!c || !out || blk < 0 || blk >= (int)c->hb.size()) return TRANS_EINVAL;
     if (!c->d_stats) return fail(c, TRANS_EINVAL, "statistics are not enabled");
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (int rc = sync_results(c)) return rc;
     return copy_view(c, blk, *out, c->d_stats, TRANS_NSTAT, false);
 }
 
@@ -175,7 +175,7 @@ int trans_hip_write_stats(trans_ctx* c, int blk, const trans_fview* xc, const tr
 {
     if (!c || !path || !xc || !yc || !zc || blk < 0 || blk >= (int)c->hb.size()) return TRANS_EINVAL;
     if (!c->d_stats) return fail(c, TRANS_EINVAL, "statistics are not enabled");
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (int rc = sync_results(c)) return rc;
     std::vector<double> st;
     int rc = pack_block(c, blk, c->d_stats, c->tot, TRANS_NSTAT, st, false);
     if (rc) return rc;

@@ -202,6 +202,10 @@ static bool srv_collect(trans_srv* s, SrvReq* r)
         const int n = r->iters + it + 1;
         if (!(g == g)) {
             r->iters = n;
+            if (const int rc = trans_hip_sync(r->ctx)) {  // an expired sweep, not the flow
+                srv_retire(s, r, TRANS_SRV_FAILED, rc);
+                return true;
+            }
             s->err = "request " + std::to_string(r->id) + ": residual is NaN at iteration " + std::to_string(n);
             srv_retire(s, r, TRANS_SRV_FAILED, TRANS_ENONFINITE);
             return true;

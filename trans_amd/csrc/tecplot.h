@@ -154,7 +154,7 @@ int trans_hip_write_tecplot(trans_ctx* c, int blk, const trans_fview* x, const t
     const size_t np = (size_t)h.ni * h.nj * h.nk;
     std::vector<double> cv((size_t)TEC_NCELLVAR * ncell), pts(3 * np);
     double* d = nullptr;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (int rc = sync_results(c)) return rc;
     HIPCHK(c, hipMalloc(&d, cv.size() * sizeof(double)));
     hipLaunchKernelGGL(k_field_vars, dim3((unsigned)((ncell + 255) / 256)), dim3(256), 0, c->stream, c->f,
                        blk_info(c, blk), c->p.omega1, s[0], s[1], s[2], s[3], d);

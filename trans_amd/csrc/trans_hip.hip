@@ -131,6 +131,7 @@ struct trans_ctx {
     int* d_tctr = nullptr;
     size_t tile_bytes = 0;
     int* d_err = nullptr;
+    bool unchecked = false;  // sweeps were queued since d_err was read
     std::vector<long> mwoff;  // per-block offset of the wall marks (size nblk+1)
     std::vector<void*> allocs;
     // time statistics (Average_Fields): TRANS_NSTAT components, allocated when enabled
@@ -298,6 +299,27 @@ static int d2h(trans_ctx* c, void* dst, const void* src, size_t bytes)
     HIPCHK(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return 0;
+}
+
+// The error flag of the wave sweeps' bounded waits (read once the stream is idle).
+static int check_sweep_flag(trans_ctx* c)
+{
+    if (!c->d_err) return 0;
+    int e = 0;
+    HIPCHK(c, hipMemcpyAsync(&e, c->d_err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->unchecked = false;
+    if (!e) return 0;
+    HIPCHK(c, hipMemsetAsync(c->d_err, 0, sizeof(int), c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return fail(c, TRANS_ETIMEOUT, "a bounded wait of the wave LU-SGS sweep expired; results are invalid");
+}
+
+// The stream's work is done and its results are valid: before anything computed is handed out.
+static int sync_results(trans_ctx* c)
+{
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return c->unchecked ? check_sweep_flag(c) : 0;
 }
 
 template <typename T>
@@ -1102,14 +1124,14 @@ int trans_hip_set_state(trans_ctx* c, int blk, const trans_state_view* s)
 int trans_hip_get_state(trans_ctx* c, int blk, const trans_state_view* s)
 {
     if (!c || !s || blk < 0 || blk >= (int)c->hb.size()) return TRANS_EINVAL;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (int rc = sync_results(c)) return rc;
     return copy_state_views(c, blk, s, false);
 }
 
 int trans_hip_get_field(trans_ctx* c, int blk, int which, const trans_fview* out)
 {
     if (!c || !out || blk < 0 || blk >= (int)c->hb.size()) return TRANS_EINVAL;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (int rc = sync_results(c)) return rc;
     Fields& f = c->f;
     switch (which) {
     case TRANS_FIELD_D: return copy_view(c, blk, *out, f.D, 7, false);
@@ -1390,6 +1412,7 @@ static void launch_wave_rule(trans_ctx* c)
 template <typename R, int NEQ>
 static void launch_wave(trans_ctx* c)
 {
+    c->unchecked = true;
     KLAUNCH(c, "k_wave_rhs", (k_wave_rhs<R, NEQ != 2, NEQ != 5>), dim3(c->seg_wtile.n), dim3(WG), c->p, c->f, c->d_blk,
             c->seg_wtile.d, c->d_tctr, (uint4*)c->wave_edge, (long)(2 * (size_t)c->edge_n * sizeof(R) / 16));
     if (c->wave_alt)
@@ -1550,19 +1573,6 @@ static int rk_update_async(trans_ctx* c, int stage)
     }
     KLAUNCH(c, "k_norm_final", k_norm_final, dim3(nblk), dim3(256), c->d_part, c->d_wrange, c->d_blk, c->d_resid);
     return launch_check(c, "rk_update");
-}
-
-// The error flag of the wave sweeps' bounded waits (read once the stream is idle).
-static int check_sweep_flag(trans_ctx* c)
-{
-    if (!c->d_err) return 0;
-    int e = 0;
-    HIPCHK(c, hipMemcpyAsync(&e, c->d_err, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (!e) return 0;
-    HIPCHK(c, hipMemsetAsync(c->d_err, 0, sizeof(int), c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return fail(c, TRANS_ETIMEOUT, "a bounded wait of the wave LU-SGS sweep expired; results are invalid");
 }
 
 static int fetch_resid(trans_ctx* c, trans_resid* per_block)
@@ -1826,6 +1836,7 @@ int trans_hip_iterate(trans_ctx* c, int n_iter, trans_resid* per_block)
         const bool replay = c->graphs && !c->plain && !c->prof && iteration_is_static(c);
         if (replay && !c->gexec && capture_iteration(c) != 0) c->graphs = false;  // eager from now on
         if (replay && c->gexec) {
+            c->unchecked = c->unchecked || c->wave;
             HIPCHK(c, hipGraphLaunch(c->gexec, c->stream));
         } else {
             drop_graph(c);
@@ -1884,7 +1895,7 @@ int trans_hip_plane_integrals(trans_ctx* c, int blk, int dir, int index, trans_p
             c->d_mon);
     double r[6];
     HIPCHK(c, hipMemcpyAsync(r, c->d_mon, sizeof(r), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (int rc = sync_results(c)) return rc;
     out->mass_flow = r[0];
     out->area = r[1];
     out->p0_mass_avg = r[2];
