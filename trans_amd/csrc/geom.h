@@ -31,10 +31,11 @@ double* wd_scratch_for_current_device()
     return wd_scratch_ptr[dev];
 }
 
-// Whether the sorted form of the wall distance pays.  It costs about 0.2 ms of sorting; every cell
-// against every panel takes at least 0.1 us per panel, the time of one workgroup: 20 000 cells and
-// 4 000 panels 664 us against 487 us sorted, 161 000 and 1 590 787 us against 867 us, 4 096 and 1 024
-// 264 us against 329 us.
+// Whether the sorted form of the wall distance pays.  It costs about 0.1 ms of sorting; every cell
+// against every panel takes at least 0.1 us per panel, the time of one workgroup.  Calls with every
+// pair and sorted: 4 096 cells and 2 048 panels 0.50 and 0.37 ms, 20 000 and 2 048 0.55 and 0.39 ms,
+// 4 096 and 30 000 3.9 and 1.8 ms, 485 000 and 2 048 2.1 and 1.0 ms; below, 4 096 and 1 024 0.26 and
+// 0.33 ms.
 bool wb_worth(long ncell, long npanel)
 {
     return npanel >= 2048 && ncell >= 4096 && ncell < (1L << 30) && npanel < (1L << 30);
@@ -48,19 +49,16 @@ void launch_wb(hipStream_t s, const double* dc, long ncell, const double* dp, lo
     double4* sc = (double4*)m;
     double4* sp = sc + ncell;
     double* tb = (double*)(sp + npanel);
-    unsigned long long* box = (unsigned long long*)(tb + 6 * (long)ntile);
-    int* bins = (int*)(box + 12);
+    double* faces = tb + 6 * (long)ntile;
+    int* bins = (int*)(faces + 6 * WB_SIDE);
     int* from = bins + 2 * WB_BINS;
-    hipLaunchKernelGGL(k_wb_clear, dim3(64), dim3(256), 0, s, box, bins);
-    const auto grid = [](long n) { return dim3((unsigned)((n + 255) / 256)); };
-    hipLaunchKernelGGL(k_wb_box, dim3(256), dim3(256), 0, s, dc, ncell, box);
-    hipLaunchKernelGGL(k_wb_box, dim3(64), dim3(256), 0, s, dp, npanel, box + 6);
-    hipLaunchKernelGGL(k_wb_count, grid(ncell), dim3(256), 0, s, dc, ncell, box, bins);
-    hipLaunchKernelGGL(k_wb_count, grid(npanel), dim3(256), 0, s, dp, npanel, box + 6, bins + WB_BINS);
+    const WbSet cells{dc, ncell, faces, bins, sc, from};
+    const WbSet panels{dp, npanel, faces + 3 * WB_SIDE, bins + WB_BINS, sp, nullptr};
+    const dim3 both((unsigned)((ncell + 255) / 256 + (npanel + 255) / 256));
+    hipLaunchKernelGGL(k_wb_faces, dim3(6 + 32), dim3(WB_SAMPLE), 0, s, cells, panels, faces);
+    hipLaunchKernelGGL(k_wb_count, both, dim3(256), 0, s, cells, panels);
     hipLaunchKernelGGL(k_wb_scan, dim3(2), dim3(1024), 0, s, bins);
-    hipLaunchKernelGGL(k_wb_scatter, grid(ncell), dim3(256), 0, s, dc, ncell, box, bins, sc, from);
-    hipLaunchKernelGGL(k_wb_scatter, grid(npanel), dim3(256), 0, s, dp, npanel, box + 6, bins + WB_BINS, sp,
-                       (int*)nullptr);
+    hipLaunchKernelGGL(k_wb_scatter, both, dim3(256), 0, s, cells, panels);
     hipLaunchKernelGGL(k_wb_tiles, dim3((unsigned)ntile), dim3(64), 0, s, sp, (int)npanel, ntile, tb);
     hipLaunchKernelGGL(k_wb_distance, dim3((unsigned)((ncell + 63) / 64)), dim3(64), 0, s, sc,
                        from, ncell, sp, (int)npanel, tb, ntile, dd);
@@ -115,7 +113,7 @@ int trans_geom_wall_distance(const double* cells, long ncell, const double* pane
     bool sorted = wb_worth(ncell, npanel);
     const long ntile = (npanel + WB_TILE - 1) / WB_TILE;
     const size_t plain = 8 * (size_t)(4 * ncell + 3 * npanel);
-    const size_t more = 32 * (size_t)(ncell + npanel) + 48 * (size_t)ntile + 4 * (size_t)ncell + 8 * 12 +
+    const size_t more = 32 * (size_t)(ncell + npanel) + 48 * (size_t)ntile + 4 * (size_t)ncell + 8 * 6 * WB_SIDE +
                         2 * WB_BINS * sizeof(int) + 256;
     char* mem = nullptr;
     if (sorted && hipMalloc(&mem, plain + more) != hipSuccess) {

@@ -296,91 +296,119 @@ __global__ void __launch_bounds__(256) k_geom_ghosts(GeomGrid g, GeomOut o)
 
 // ---------------------------------------------------------------------------------------
 // The same minimum over fewer pairs, for many points: cells and panels are put in Morton order
-// (32^3 boxes of their bounding box, counting sort), panels in tiles of 64 with their bounding
+// (32^3 boxes, counting sort), panels in tiles of 64 with their bounding
 // boxes.  A wave holds 64 consecutive cells; it evaluates the tile that is nearest to
 // its cells' box, then every tile whose box is not farther than its largest minimum so far from its
 // cells' box, and then not farther from some cell than that cell's minimum.  A
 // skipped tile's pairs are all above the minima by more than their rounding (WB_SLACK), the pairs
 // evaluated are formed as above, and a minimum does not depend on the order, so the result is the
-// same bit for bit.  485 000 cells and 30 000 panels: 1.1 ms of kernels and 2.5 ms for the call, with
-// every pair 6 ms and 7.7 ms.  With two and four cells per lane 1.3 and 1.6 ms (larger boxes).
-constexpr int WB_BITS = 5, WB_BINS = 1 << (3 * WB_BITS);
+// same bit for bit.  485 000 cells and 30 000 panels: 1.2 ms of kernels and 2.0 ms for the call, with
+// every pair 6 ms and 7.9 ms.  With two and four cells per lane the last kernel took 1.3 and 1.6 ms
+// instead of 1.1 ms (larger boxes).
+//
+// The boxes' faces are quantiles of the coordinates, taken from a sample, so that each slab holds
+// about 1/32 of the points however they are spread.  Equal boxes of the bounding box put nearly all
+// points into one where a single point was far away.  Calls with equal boxes, and now (with every
+// pair): 485 000 x 30 000 with one far cell 18.5 ms, 2.0 ms (8.0 ms); 485 000 x 2 048 with a far cell
+// and a far panel 12.6 ms, 1.1 ms (2.1 ms); an O-grid stretched to 100 chords, 512 000 x 20 480,
+// 3.2 ms, 1.9 ms (6.4 ms); 100 000 x 10 000 coincident points 4.6 ms, 1.8 ms (2.0 ms).  What is still
+// slower than every pair is a set none of whose panels is nearer than another: 485 000 cells on the
+// axis of a cylinder of 30 000 panels 8.9 ms (7.6 ms).
+constexpr int WB_BITS = 5, WB_SIDE = 1 << WB_BITS, WB_BINS = 1 << (3 * WB_BITS);
 constexpr int WB_TILE = 64;
+constexpr int WB_SAMPLE = 512;
 constexpr double WB_SLACK = 1.0 + 1.0e-9;
 
-// Doubles as unsigned integers of the same order, for atomic minima and maxima.
-__device__ __forceinline__ unsigned long long wb_key(double x)
-{
-    const unsigned long long u = (unsigned long long)__double_as_longlong(x);
-    return u >> 63 ? ~u : u | (1ull << 63);
-}
-__device__ __forceinline__ double wb_unkey(unsigned long long u)
-{
-    return __longlong_as_double((long long)(u >> 63 ? u & ~(1ull << 63) : ~u));
-}
+// A set of points in sorted form, and its tables.
+struct WbSet {
+    const double* pt;  // x, then y, then z of all points
+    long n;
+    const double* faces;  // 3 x WB_SIDE
+    int* bins;
+    double4* out;  // x, y, z, 0 per point, in order
+    int* from;     // where a point came from, or null
+};
 
-// Two boxes (cells, panels) and their tables before the first point.
-__global__ void __launch_bounds__(256) k_wb_clear(unsigned long long* __restrict__ box, int* __restrict__ bins)
+// The faces between the slabs, one workgroup per set of points and coordinate (0 to 5): entry k of
+// the 32 is the lower face of slab k (entry 0 is not used).  The sample is one point of each of
+// WB_SAMPLE equal runs of the points, at a scattered place, so that the strides of a grid do not
+// show in it.  The other workgroups clear the tables.
+__global__ void __launch_bounds__(WB_SAMPLE) k_wb_faces(WbSet cells, WbSet panels, double* __restrict__ faces)
 {
-    const int q = blockIdx.x * 256 + threadIdx.x;
-    for (int k = q; k < 2 * WB_BINS; k += gridDim.x * 256) bins[k] = 0;
-    if (q < 12) box[q] = q % 6 < 3 ? ~0ull : 0ull;
-}
-
-// box: keys of the lower corner (3, initially all ones), then of the upper one (3, initially zero)
-__global__ void __launch_bounds__(256) k_wb_box(const double* __restrict__ pt, long n, unsigned long long* box)
-{
-    double lo[3], hi[3];
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-        lo[d] = INFINITY;
-        hi[d] = -INFINITY;
+    const int t = threadIdx.x;
+    if (blockIdx.x >= 6) {
+        int* const bins = cells.bins;  // (the panels' behind them)
+        for (int k = (blockIdx.x - 6) * WB_SAMPLE + t; k < 2 * WB_BINS; k += (gridDim.x - 6) * WB_SAMPLE) bins[k] = 0;
+        return;
     }
-    for (long q = (long)blockIdx.x * 256 + threadIdx.x; q < n; q += (long)gridDim.x * 256)
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            const double x = pt[d * n + q];
-            if (!isfinite(x)) continue;
-            lo[d] = fmin(lo[d], x);
-            hi[d] = fmax(hi[d], x);
-        }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            lo[d] = fmin(lo[d], __shfl_xor(lo[d], off, 64));
-            hi[d] = fmax(hi[d], __shfl_xor(hi[d], off, 64));
-        }
-    if (threadIdx.x % 64 == 0)
-#pragma unroll
-        for (int d = 0; d < 3; d++)
-            if (lo[d] <= hi[d]) {
-                atomicMin(box + d, wb_key(lo[d]));
-                atomicMax(box + 3 + d, wb_key(hi[d]));
+    __shared__ double x[WB_SAMPLE];
+    const WbSet& s = blockIdx.x < 3 ? cells : panels;
+    const long from = s.n * t / WB_SAMPLE, len = max(1L, s.n * (t + 1) / WB_SAMPLE - from);
+    const double v = s.pt[blockIdx.x % 3 * s.n + from + (long)((unsigned)t * 2654435761u >> 8) % len];
+    x[t] = v != v ? INFINITY : v;  // (a NaN has no place in an order)
+    // bitonic sort
+    for (int k = 2; k <= WB_SAMPLE; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            __syncthreads();
+            const int o = t ^ j;
+            if (o > t) {
+                const double a = x[t], b = x[o];
+                if ((a > b) == ((t & k) == 0)) {
+                    x[t] = b;
+                    x[o] = a;
+                }
             }
+        }
+    __syncthreads();
+    if (t < WB_SIDE) faces[blockIdx.x * WB_SIDE + t] = x[t * (WB_SAMPLE / WB_SIDE)];
 }
 
-// Morton number of point q among the boxes of the bounding box.
-__device__ __forceinline__ int wb_bin(const double* __restrict__ pt, long n, long q, const unsigned long long* box)
+// The set that a workgroup takes 256 points of, and the first of them: the cells, then the panels.
+__device__ __forceinline__ const WbSet& wb_share(const WbSet& cells, const WbSet& panels, long& base)
+{
+    const long nc = (cells.n + 255) / 256;
+    base = ((long)blockIdx.x < nc ? (long)blockIdx.x : (long)blockIdx.x - nc) * 256;
+    return (long)blockIdx.x < nc ? cells : panels;
+}
+
+// Morton number of point q among the boxes; faces: of its set of points, in LDS.
+__device__ __forceinline__ int wb_bin(const double* __restrict__ pt, long n, long q, const double* faces)
 {
     int m = 0;
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-        const double lo = wb_unkey(box[d]), hi = wb_unkey(box[3 + d]);
-        const double s = (pt[d * n + q] - lo) / (hi - lo) * (1 << WB_BITS);
-        // (NaN, of a coordinate or of a flat box, takes the first)
-        const int k = (int)fmin(fmax(s, 0.0), (double)((1 << WB_BITS) - 1));
+        const double x = pt[d * n + q];
+        int k = 0;  // (of a NaN too)
+#pragma unroll
+        for (int s = WB_SIDE / 2; s > 0; s >>= 1) k += x >= faces[d * WB_SIDE + k + s] ? s : 0;
 #pragma unroll
         for (int b = 0; b < WB_BITS; b++) m |= ((k >> b) & 1) << (3 * b + d);
     }
     return m;
 }
 
-__global__ void __launch_bounds__(256) k_wb_count(const double* __restrict__ pt, long n,
-                                                  const unsigned long long* __restrict__ box, int* __restrict__ bins)
+// Adds 1 to counter `m` for every active lane and returns the lane's place.  The lanes that share
+// the first lane's counter, of which there are many where points coincide, add theirs together.
+__device__ __forceinline__ int wb_add(int* __restrict__ bins, int m)
 {
-    const long q = (long)blockIdx.x * 256 + threadIdx.x;
-    if (q < n) atomicAdd(bins + wb_bin(pt, n, q, box), 1);
+    const int lead = __builtin_amdgcn_readfirstlane(m);
+    const unsigned long long same = __ballot(m == lead);
+    if (m != lead) return atomicAdd(bins + m, 1);
+    const int before = __popcll(same & ((1ull << (threadIdx.x & 63)) - 1));
+    int at = 0;
+    if (before == 0) at = atomicAdd(bins + m, __popcll(same));
+    return __builtin_amdgcn_readfirstlane(at) + before;
+}
+
+__global__ void __launch_bounds__(256) k_wb_count(WbSet cells, WbSet panels)
+{
+    __shared__ double s_faces[3 * WB_SIDE];
+    long base;
+    const WbSet& s = wb_share(cells, panels, base);
+    if (threadIdx.x < 3 * WB_SIDE) s_faces[threadIdx.x] = s.faces[threadIdx.x];
+    __syncthreads();
+    const long q = base + threadIdx.x;
+    if (q < s.n) (void)wb_add(s.bins, wb_bin(s.pt, s.n, q, s_faces));
 }
 
 // Counts to first positions; one workgroup per table.
@@ -407,17 +435,19 @@ __global__ void __launch_bounds__(1024) k_wb_scan(int* __restrict__ tables)
     }
 }
 
-// Points to their sorted places: x, y, z, 0 per point, and where they came from (if asked for).
-__global__ void __launch_bounds__(256) k_wb_scatter(const double* __restrict__ pt, long n,
-                                                    const unsigned long long* __restrict__ box,
-                                                    int* __restrict__ bins, double4* __restrict__ out,
-                                                    int* __restrict__ from)
+// Points to their sorted places.
+__global__ void __launch_bounds__(256) k_wb_scatter(WbSet cells, WbSet panels)
 {
-    const long q = (long)blockIdx.x * 256 + threadIdx.x;
-    if (q >= n) return;
-    const int at = atomicAdd(bins + wb_bin(pt, n, q, box), 1);
-    out[at] = make_double4(pt[q], pt[n + q], pt[2 * n + q], 0.0);
-    if (from) from[at] = (int)q;
+    __shared__ double s_faces[3 * WB_SIDE];
+    long base;
+    const WbSet& s = wb_share(cells, panels, base);
+    if (threadIdx.x < 3 * WB_SIDE) s_faces[threadIdx.x] = s.faces[threadIdx.x];
+    __syncthreads();
+    const long q = base + threadIdx.x;
+    if (q >= s.n) return;
+    const int at = wb_add(s.bins, wb_bin(s.pt, s.n, q, s_faces));
+    s.out[at] = make_double4(s.pt[q], s.pt[s.n + q], s.pt[2 * s.n + q], 0.0);
+    if (s.from) s.from[at] = (int)q;
 }
 
 // Bounding boxes of the panel tiles: 3 lower, 3 upper bounds, each ntile values; one wave per tile.
