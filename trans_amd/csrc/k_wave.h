@@ -12,8 +12,10 @@
 // edge value is its own flag: the buffers are filled with a NaN pattern before the sweeps
 // (k_wave_rhs), a consumer loads its values PD rows ahead and, where a loaded value still
 // is that pattern, polls until the producer has stored it.  There are no progress counters,
-// no chunks and no waits for stores to complete; each value is one 4- or 8-byte agent-scope
-// word, so no order between stores matters.  Tiles are work items taken from an atomic
+// no chunks and no waits for stores to complete; each value is in one aligned 8-byte word that
+// is stored and loaded at agent scope (two FP32 values, each its own flag, or one FP64 value, which
+// must arrive whole: these are the instructions and cache bits of a relaxed 64-bit atomic load or
+// store), so no order between stores matters.  Tiles are work items taken from an atomic
 // counter with a tile's upstream tiles first, so a wait is always for a tile that has started;
 // every wait is bounded (spin_limit), past it the error flag is raised and the sweep goes on.
 //
@@ -41,7 +43,10 @@
 
 constexpr int WVA = 16, WVB = 4;            // lines of a tile along i and along k
 constexpr int WV_SKEW = WVA - 1 + WVB - 1;  // rows a tile has beyond NJ1
-constexpr unsigned WV_SENTINEL = 0xFFF5A5A5u;  // (each half of) an edge value not yet stored: a NaN no operation makes
+// (Each half of) an edge value not yet stored: a NaN that no operation makes of other values.  In
+// FP32 operations hand it on, so a tile that gave up a wait may store it as a value; its neighbours
+// then count it as missing, until their waits end by the error flag.
+constexpr unsigned WV_SENTINEL = 0xFFF5A5A5u;
 constexpr int WV_SPIN_LIMIT = 1 << 18;      // polls of one bounded wait (about 0.3 s)
 
 // Values of one lane in a packet row.  The face means and the spectral radii are stored halved
@@ -70,8 +75,9 @@ struct WaveRow {
 };
 
 // Edge row: what the lanes on a tile's outgoing i and k faces hand on at one row, as 8-byte words per
-// lane (one FP64 value, or two FP32 values of which the last may be padding): byte offsets.  16-byte
-// words (3 to 5 % faster on small grids) gave results that differed from run to run.
+// lane (one FP64 value, or two FP32 values of which the last may be padding): byte offsets.  (16-byte
+// words, 3 to 5 % faster on small grids, gave results that differed from run to run: nothing promises
+// that such a word arrives whole.)
 template <typename R>
 struct WaveEdge {
     static constexpr int ELEMS = 160;
@@ -566,8 +572,8 @@ __device__ __forceinline__ void wave_sweep(const Fields& f, const BlkInfo& b, in
         constexpr int Q = decltype(qc)::value;
         WaveIn<R, NEQ>& x = ring[Q];
         // the row's loads are complete: what may still be in flight are the operations issued
-        // after them, the stores of their step and whole steps since (the compiler's own counter
-        // waits were found missing where a ring of three rows crosses the loop's end)
+        // after them, the stores of their step and whole steps since.  (A test follows every load
+        // through the assembly; the compiler's own waits alone passed it too.)
         __builtin_amdgcn_s_waitcnt(wv_vmcnt(NST + (PD - 1) * (NLD + NST)));
         __builtin_amdgcn_sched_barrier(0);
         // the i terms from the row's previous lanes; the first lane of a DPP row keeps its edge value
