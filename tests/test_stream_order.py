@@ -51,11 +51,3 @@ def test_failed_launch_leaves_nothing_unordered(stub, kind, call):
         assert not _unjoined(events(stub), main), q
     stub.stub_reset()
     sv.close()
-
-
-def test_a_context_has_one_helper_stream(stub):
-    blocks, prm = _case("plate")
-    stub.stub_reset()
-    sv = Solver(blocks, prm, ki=1)
-    assert sum(what == "stream" for what, _, _ in events(stub)) == 2
-    sv.close()

@@ -95,11 +95,11 @@ struct trans_ctx {
     trans_resid* d_resid = nullptr;
     double* d_mon = nullptr;  // 6 doubles: result of k_plane_integrals
     hipStream_t stream = nullptr;
-    // helper stream for independent kernels of one call (forked from and joined back
+    // helper streams for independent kernels of one call (forked from and joined back
     // into `stream` inside the call, so that calls stay ordered on `stream`)
-    hipStream_t aux = nullptr;      // `stream` itself while one stream is used
-    hipStream_t aux_own = nullptr;  // the created one (null: single-stream context)
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    hipStream_t aux[3] = {nullptr, nullptr, nullptr};
+    hipStream_t aux_own[3] = {nullptr, nullptr, nullptr};  // created helper streams (null: single-stream context)
+    hipEvent_t ev_fork = nullptr, ev_join[3] = {nullptr, nullptr, nullptr};
     // one outer iteration captured as a HIP graph and replayed while the iteration's kernel
     // arguments stay the same (set_params and profiling drop it)
     bool graphs = true;
@@ -234,23 +234,25 @@ static int no_host_memory(trans_ctx* c)
     return TRANS_ENOMEM;
 }
 
-// The helper stream waits for the work queued so far on the context's stream.
-static void fork_aux(trans_ctx* c)
+// Helper streams 0..n-1 wait for the work queued so far on the context's stream.
+static void fork_aux(trans_ctx* c, int n)
 {
-    if (c->aux == c->stream) return;
+    if (c->aux[0] == c->stream) return;  // single-stream context
     (void)hipEventRecord(c->ev_fork, c->stream);
-    (void)hipStreamWaitEvent(c->aux, c->ev_fork, 0);
+    for (int q = 0; q < n; q++) (void)hipStreamWaitEvent(c->aux[q], c->ev_fork, 0);
 }
 
-// The context's stream waits for the work queued on the helper stream.
-static void join_aux(trans_ctx* c)
+// The context's stream waits for the work queued on helper streams 0..n-1.
+static void join_aux(trans_ctx* c, int n)
 {
-    if (c->aux == c->stream) return;
-    (void)hipEventRecord(c->ev_join, c->aux);
-    (void)hipStreamWaitEvent(c->stream, c->ev_join, 0);
+    if (c->aux[0] == c->stream) return;
+    for (int q = 0; q < n; q++) {
+        (void)hipEventRecord(c->ev_join[q], c->aux[q]);
+        (void)hipStreamWaitEvent(c->stream, c->ev_join[q], 0);
+    }
 }
 
-// A fork of the helper stream that is joined on every way out.
+// A fork of helper stream 0 that is joined on every way out.
 struct AuxScope {
     trans_ctx* c;
     bool open = false;
@@ -258,12 +260,12 @@ struct AuxScope {
     ~AuxScope() { join(); }
     void fork()
     {
-        fork_aux(c);
+        fork_aux(c, 1);
         open = true;
     }
     void join()
     {
-        if (open) join_aux(c);
+        if (open) join_aux(c, 1);
         open = false;
     }
 };
@@ -675,7 +677,7 @@ static int set_sweep(trans_ctx* c, int m, bool upload)
     return fail(c, TRANS_EHIP, std::string("face means: ") + hipGetErrorString(e));
 }
 
-// dry: sizing run only.  single_stream: the helper stream is the context's own stream, so
+// dry: sizing run only.  single_stream: the helper streams are the context's own stream, so
 // that every launch of the context is ordered on one stream (the serving layer's contexts:
 // one stream each spreads the resident solves over the device's hardware queues).
 static int create_ctx(const trans_params* params, int nblk, const trans_block_desc* blocks, trans_ctx** out,
@@ -718,13 +720,16 @@ static int create_ctx(const trans_params* params, int nblk, const trans_block_de
         }
     if (!dry) {
         HIPCHK(c, hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-        c->aux = c->stream;
-        if (!single_stream) {
-            HIPCHK(c, hipStreamCreateWithFlags(&c->aux_own, hipStreamNonBlocking));
-            c->aux = c->aux_own;
-            HIPCHK(c, hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
-            HIPCHK(c, hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
+        for (int q = 0; q < 3; q++) {
+            if (single_stream) {
+                c->aux[q] = c->stream;
+                continue;
+            }
+            HIPCHK(c, hipStreamCreateWithFlags(&c->aux_own[q], hipStreamNonBlocking));
+            c->aux[q] = c->aux_own[q];
+            HIPCHK(c, hipEventCreateWithFlags(&c->ev_join[q], hipEventDisableTiming));
         }
+        if (!single_stream) HIPCHK(c, hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
     }
     {
         const char* env = std::getenv("TRANS_HIP_GRAPH");
@@ -901,8 +906,10 @@ int trans_hip_destroy(trans_ctx* c)
     free_tiles(c);
     if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
     if (c->graph) (void)hipGraphDestroy(c->graph);
-    if (c->aux_own) (void)hipStreamDestroy(c->aux_own);
-    if (c->ev_join) (void)hipEventDestroy(c->ev_join);
+    for (int q = 0; q < 3; q++) {
+        if (c->aux_own[q]) (void)hipStreamDestroy(c->aux_own[q]);
+        if (c->ev_join[q]) (void)hipEventDestroy(c->ev_join[q]);
+    }
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -1263,7 +1270,7 @@ static int space_async(trans_ctx* c, bool prim)
     AuxScope aux(c);
     auto conv_aside = [&]() {
         aux.fork();
-        launch_conv(c, c->aux, if_turb, 0, nblk);
+        launch_conv(c, c->aux[0], if_turb, 0, nblk);
     };
     if (side && early) conv_aside();
     if (visc) {
@@ -1307,7 +1314,7 @@ int trans_hip_residual(trans_ctx* c)
     AuxScope aux(c);
     if (c->n_outl) {
         aux.fork();
-        KLAUNCH_ON(c, c->aux, "k_bc_outlet", k_bc_outlet, dim3(c->n_outl), dim3(256), c->p, if_turb_now(c), c->f,
+        KLAUNCH_ON(c, c->aux[0], "k_bc_outlet", k_bc_outlet, dim3(c->n_outl), dim3(256), c->p, if_turb_now(c), c->f,
                    c->d_blk, c->d_patch, c->d_outl);
     }
     KLAUNCH(c, "k_spectral_radius", k_spectral_radius<true>, dim3(c->seg_cell.n), dim3(WG), c->p, c->ki,

@@ -7,15 +7,14 @@
 //   - the LU-SGS sweep: the tile wavefront along j, the line march along i or k where the cross
 //     sections fit one workgroup, one launch per hyperplane, or the one-workgroup hyperplane
 //     kernel;
-//   - the helper stream (convective faces beside the gradients or the viscous faces, the outlet
-//     march beside the spectral radius) or one stream;
+//   - the helper streams (face kernels of the three directions concurrently) or one stream;
 //   - replaying the iteration as a HIP graph or launching it eagerly.
 // Each candidate runs `iters` timed iterations from the same saved state (after one untimed
 // iteration that also captures its graph); the fastest is kept and the state restored.
 
 static void apply_streams(trans_ctx* c, bool single)
 {
-    c->aux = single || !c->aux_own ? c->stream : c->aux_own;
+    for (int q = 0; q < 3; q++) c->aux[q] = (single || !c->aux_own[q]) ? c->stream : c->aux_own[q];
     drop_graph(c);
 }
 
@@ -53,7 +52,7 @@ int trans_hip_autotune(trans_ctx* c, int iters, trans_tune_entry* out, int max_o
     const bool plain0 = c->plain;
     c->plain = false;
     const int sweep0 = plain0 ? -2 : cur_sweep(c);
-    const bool single0 = c->aux == c->stream;
+    const bool single0 = c->aux[0] == c->stream;
     c->stats_on = false;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     int rc = copy_state(false);
@@ -73,7 +72,7 @@ int trans_hip_autotune(trans_ctx* c, int iters, trans_tune_entry* out, int max_o
         if (rc) break;
         if (cur_sweep(c) != sw) continue;  // it runs one launch per hyperplane, a candidate of its own
         for (int st = 0; st < 2 && !rc; st++) {
-            if (st == 0 && !c->aux_own) continue;  // single-stream context
+            if (st == 0 && !c->aux_own[0]) continue;  // single-stream context
             apply_streams(c, st == 1);
             for (int g = 0; g < 2 && !rc; g++) {
                 c->graphs = g == 1;
@@ -147,7 +146,7 @@ int trans_hip_set_tuning(trans_ctx* c, const trans_tune_entry* t)
     }
     c->plain = false;
     if (t->streams != 1 && t->streams != 4) return fail(c, TRANS_EINVAL, "streams must be 1 or 4");
-    if (t->streams == 4 && !c->aux_own) return fail(c, TRANS_EINVAL, "this context has one stream");
+    if (t->streams == 4 && !c->aux_own[0]) return fail(c, TRANS_EINVAL, "this context has one stream");
     if (t->sweep == 3 && (t->tile_a < 1 || t->tile_b < 1 || t->tile_a * t->tile_b > 256 || t->chunk < 1))
         return fail(c, TRANS_EINVAL, "tile shape must have 1..256 lines and chunk >= 1");
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -171,7 +170,7 @@ int trans_hip_get_tuning(const trans_ctx* c, trans_tune_entry* out)
 {
     if (!c || !out) return TRANS_EINVAL;
     out->sweep = cur_sweep(c);
-    out->streams = c->aux == c->stream ? 1 : 4;
+    out->streams = c->aux[0] == c->stream ? 1 : 4;
     out->graph = c->graphs ? 1 : 0;
     out->ms_per_iter = 0.0;
     out->tile_a = c->tile_a;
