@@ -50,3 +50,23 @@ def test_failed_allocations_free_what_they_took(stub):
             sv.set_tuning(3, 1, 0)
         assert stub.stub_mapped() == before
     sv.close()
+
+
+def test_refused_configuration_changes_nothing(stub):
+    blocks, org, glob = cases.flat_plate(nblk=1, ni_total=70, nj=35, nk=34, lo=9, hi=70)  # no axis fits a line march
+    sv = Solver(blocks, solver.prepare_case(blocks, org, glob), ki=1)
+    for keep in ((-3, 1, 0), (3, 4, 1), (-2, 1, 0)):
+        sv.set_tuning(*keep)
+        stub.stub_reset()
+        sv.iterate(1)
+        was = sv.tuning()
+        launches = events(stub)
+        for bad in ((3, 2, 0), (5, 1, 0), (0, 1, 0), (1, 4, 0), (3, 4, 0, 0, 1, 8)):
+            with pytest.raises(TransError) as e:
+                sv.set_tuning(*bad)
+            assert e.value.rc == capi.TRANS_EINVAL
+            assert sv.tuning() == was, (keep, bad)
+            stub.stub_reset()
+            sv.iterate(1)
+            assert [x[:2] for x in events(stub) if x[0] == "launch"] == [x[:2] for x in launches if x[0] == "launch"]
+    sv.close()

@@ -7,7 +7,8 @@
 //   - the LU-SGS sweep: the tile wavefront along j, the line march along i or k where the cross
 //     sections fit one workgroup, one launch per hyperplane, or the one-workgroup hyperplane
 //     kernel;
-//   - the helper streams (face kernels of the three directions concurrently) or one stream;
+//   - a helper stream (convective faces beside the gradients or the viscous faces, the outlet march
+//     beside the spectral radius) or one stream;
 //   - replaying the iteration as a HIP graph or launching it eagerly.
 // Each candidate runs `iters` timed iterations from the same saved state (after one untimed
 // iteration that also captures its graph); the fastest is kept and the state restored.
@@ -144,21 +145,20 @@ int trans_hip_set_tuning(trans_ctx* c, const trans_tune_entry* t)
         drop_graph(c);
         return 0;
     }
-    c->plain = false;
     if (t->streams != 1 && t->streams != 4) return fail(c, TRANS_EINVAL, "streams must be 1 or 4");
     if (t->streams == 4 && !c->aux_own[0]) return fail(c, TRANS_EINVAL, "this context has one stream");
     if (t->sweep == 3 && (t->tile_a < 1 || t->tile_b < 1 || t->tile_a * t->tile_b > 256 || t->chunk < 1))
         return fail(c, TRANS_EINVAL, "tile shape must have 1..256 lines and chunk >= 1");
     HIPCHK(c, hipStreamSynchronize(c->stream));
     const int cur = cur_sweep(c);
+    if (t->sweep != cur) {
+        int rc = set_sweep(c, t->sweep, true);
+        if (rc) return rc;
+    }
     if (t->sweep == 3) {
         c->tile_a = t->tile_a;
         c->tile_b = t->tile_b;
         c->tile_chunk = t->chunk;
-    }
-    if (t->sweep != cur) {
-        int rc = set_sweep(c, t->sweep, true);
-        if (rc) return rc;
     }
     apply_streams(c, t->streams == 1);
     c->graphs = t->graph != 0;
