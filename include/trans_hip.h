@@ -313,8 +313,8 @@ int trans_tecplot_write_ascii(const char* path, const char* title, const char* z
  * state and keeps the fastest: the LU-SGS sweep (sweep = 0, 2: line march along i or k, where the
  * cross sections fit one workgroup; 1, where the (i, k) sections do, and 3, for all blocks: the
  * wavefront of tiles of lines along j; -2: one launch per hyperplane over all
- * blocks; -1: one workgroup per block walking its hyperplanes), helper streams for the
- * face kernels (streams = 4) or one stream (1), HIP-graph replay (graph = 1) or eager launches.
+ * blocks; -1: one workgroup per block walking its hyperplanes), a helper stream for
+ * independent kernels (streams = 4) or one stream (1), HIP-graph replay (graph = 1) or eager launches.
  * Every configuration computes the same iteration (the sweep variants contract multiply-adds
  * in different places, so they agree within rounding, not bitwise).  The state and KI are restored;
  * out (max_out entries, may be NULL) receives the timings, *n_out their count.  The sweep

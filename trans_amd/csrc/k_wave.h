@@ -26,10 +26,11 @@
 // store is dropped; with zero inputs such a lane hands zero terms on, which is what its
 // neighbours need before their first cell.
 //
-// What bounds it: a tile's rows follow each other and a row is about 200 dependent FP64
-// instructions (0.36 us; FP32 0.25 us), so with few tiles (fewer than four per SIMD) the chain
-// (NJ1 + tile diagonals x the skew) x row time; with many, the memory system (144 B/cell FP32 per
-// sweep).  Forward and backward sweep together, before (one workgroup per block marching lines
+// What bounds it: a tile's rows follow each other.  A row of the mean flow is 190 instructions in FP64,
+// 108 of them arithmetic and 36 memory operations, and takes 0.54 to 0.58 us (sweeps of 194 and 198
+// rows); 175, 108 and 21 in FP32, 0.49 us (115 rows).  So with few tiles (fewer than four per SIMD) the
+// chain (NJ1 + tile diagonals x the skew) x row time; with many, the memory system (144 B/cell FP32
+// per sweep).  Forward and backward sweep together, before (one workgroup per block marching lines
 // with a barrier per step, or tiles of 256 lines with progress counters) and now:
 //     65k-cell bump channel, FP64           707 us   218 us
 //     131k-cell plate, FP64 k-omega         406 us   225 us

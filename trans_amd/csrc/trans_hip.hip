@@ -96,7 +96,10 @@ struct trans_ctx {
     double* d_mon = nullptr;  // 6 doubles: result of k_plane_integrals
     hipStream_t stream = nullptr;
     // helper streams for independent kernels of one call (forked from and joined back
-    // into `stream` inside the call, so that calls stay ordered on `stream`)
+    // into `stream` inside the call, so that calls stay ordered on `stream`).  Work goes to the first
+    // only; the others keep a context's streams at four, one per hardware queue: with two, other
+    // contexts' streams fall on the queues unevenly (a server of four small solves beside a
+    // resident solver: 115 ms instead of 101 ms)
     hipStream_t aux[3] = {nullptr, nullptr, nullptr};
     hipStream_t aux_own[3] = {nullptr, nullptr, nullptr};  // created helper streams (null: single-stream context)
     hipEvent_t ev_fork = nullptr, ev_join[3] = {nullptr, nullptr, nullptr};
@@ -1264,7 +1267,8 @@ static int space_async(trans_ctx* c, bool prim)
     // The convective faces, bound by instruction issue, run on a helper stream beside the gradients
     // (bound by memory) and BC(0); schemes that read the shock sensor or Fscheme, beside BC(0) and
     // the viscous faces.  Per iteration 1685 -> 1615 us (0.30M-cell cascade) and 487 -> 465 us
-    // (131k-cell plate) with MDCD, 806 -> 801 us (0.49M-cell sector) with MUSCL.
+    // (131k-cell plate) with MDCD; with MUSCL no difference beyond the runs' own (806 and 801 us at
+    // 0.49M cells, 8.37 and 8.33 ms at 8.1M).
     const bool side = visc && !fused;
     const bool early = c->p.kind_spatial <= 2 && c->p.kind_roe != 2;
     AuxScope aux(c);
@@ -1396,10 +1400,11 @@ static void launch_wave_sweeps(trans_ctx* c)
 }
 
 // From four tiles per CU on (1024) the FP32 sweeps keep four rows of a wave in flight at two waves
-// per SIMD: 1169 us for both sweeps of the 8.1M-cell sector (1760 tiles, k-omega) instead of
-// 1307 us with two rows at four waves.  Below, a row's latency counts more than its loads: 179 us
-// against 201 us at 0.49M cells (392 tiles), 132 us against 134 us on a 25 k-cell plate (25 tiles)
-// (all while a poll waited for one row only; 1060, 164 and 115 us since).
+// per SIMD; below, a row's latency counts more than its loads, and they keep two at four waves.  Both
+// sweeps of compressor sectors with four rows and with two (k-omega): 206 and 165 us with 392 tiles,
+// 386 and 331 us with 700, 571 and 497 us with 1008, 693 and 684 us with 1274, 902 and 1016 us with
+// 1650, 1065 and 1231 us with 1760 (8.1M cells).  They cross at about 1300 tiles, so that between
+// 1024 and there two rows would be up to a tenth faster.
 // The FP64 k-omega sweeps alone have the registers for a third row (334 us against 414 us for the
 // three stages of a 0.30M-cell cascade); with the mean flow two rows are as good (103 us against
 // 113 us at 0.13M cells).
